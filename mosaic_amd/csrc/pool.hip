@@ -2,11 +2,12 @@
 //
 // Replaces reduce(x, 'b (nb bs) h d -> b nb h d', 'mean') (primitives.py:65-66,76): fp32
 // sum over the block's tokens in token order, divided by the block size, rounded to bf16.
-// One workgroup per (pooled block t, batch b) reads the block's q, k and v rows once
-// (HBM-bound).  Each thread streams one 16-byte column chunk down the block's tokens, summing in
-// token order; with RoPE two adjacent threads share a chunk, each taking one half of the
-// tokens, and their partial sums are added through a lane swap, which spreads the rotation
-// arithmetic over twice as many waves.
+// The workgroups of (pooled block t, batch b), one or a few that share its columns, read the
+// block's q, k and v rows once (HBM-bound).  TPC adjacent threads share one 16-byte column chunk
+// of a row: each streams it down its own contiguous run of the block's tokens, summing in token
+// order, and the partial sums are added pairwise through DPP.  More threads per chunk shorten
+// the serial walk and put more loads in flight where the grid alone leaves the chip idle
+// (pool_shape).
 // Outputs: [B, nb, H, 64] for the pooled tensors and, for k and v, the MFMA-operand-ordered
 // layouts read by the compressed-attention kernel (kfrag_index / vfrag_index; zero for the
 // padding blocks nb .. nb_pad-1).
@@ -18,6 +19,8 @@
 // pair m = (2m, 2m+1) of a head becomes (x0 c_m - x1 s_m, x1 c_m + x0 s_m), each product and
 // the sum rounded as the reference rounds them.  The rotated rows are written out (the
 // attention reads them) and pooled, so the rotation costs no extra read of q and k.
+#include <algorithm>
+
 #include "bsa_common.h"
 
 namespace mosaic {
@@ -30,14 +33,29 @@ __device__ __forceinline__ T sel3(const T (&a)[3], int which) {
     return which == 0 ? a[0] : (which == 1 ? a[1] : a[2]);
 }
 
-// x of the other lane of the pair (l, l ^ 1): DPP quad_perm [1, 0, 3, 2]
-__device__ __forceinline__ float swap_pair(float x) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0xb1, 0xf, 0xf, false));
+// x of lane l ^ 1 (quad_perm [1, 0, 3, 2]), of lane l ^ 2 (quad_perm [2, 3, 0, 1]) and of the
+// mirror lane in the group of eight (row_half_mirror)
+template <int STEP>
+__device__ __forceinline__ float other_lane(float x) {
+    constexpr int kCtrl = STEP == 1 ? 0xb1 : STEP == 2 ? 0x4e : 0x141;
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), kCtrl, 0xf, 0xf, false));
 }
-// (first half) + (second half) in both lanes of a pair, in that order (half = this lane's half)
-__device__ __forceinline__ float acc_pair(float x, int half) {
-    const float y = swap_pair(x);
-    return half ? y + x : x + y;
+// Sum (maximum) over the TPC lanes of a chunk, the same value in all of them: at each step the
+// lanes of a half all hold that half's value, so the mirror lane is as good as l ^ 4.
+// Addition is commutative, so both halves round alike.
+template <int TPC>
+__device__ __forceinline__ float chunk_add(float x) {
+    if constexpr (TPC > 1) x += other_lane<1>(x);
+    if constexpr (TPC > 2) x += other_lane<2>(x);
+    if constexpr (TPC > 4) x += other_lane<4>(x);
+    return x;
+}
+template <int TPC>
+__device__ __forceinline__ float chunk_max(float x) {
+    if constexpr (TPC > 1) x = fmaxf(x, other_lane<1>(x));
+    if constexpr (TPC > 2) x = fmaxf(x, other_lane<2>(x));
+    if constexpr (TPC > 4) x = fmaxf(x, other_lane<4>(x));
+    return x;
 }
 
 // ROPE: 0 no rotation; 1 rotation with the block's table rows staged in LDS; 2 rotation with
@@ -46,10 +64,8 @@ __device__ __forceinline__ float acc_pair(float x, int half) {
 // address spaces compiled to generic loads).
 template <int ROPE>
 constexpr int kPoolMaxThreads = ROPE == 2 ? 512 : 1024;  // the global-table variant needs more registers
-template <int ROPE>
-constexpr int kThreadsPerChunk = ROPE != 0 ? 2 : 1;
 
-template <int ROPE>
+template <int ROPE, int TPC>
 __global__ __launch_bounds__(kPoolMaxThreads<ROPE>) void pool_kernel(PoolParams p) {
     const int t = blockIdx.x, b = blockIdx.y;
     // RoPE tables of the block's tokens, read once per workgroup: [token][8 float4] of cos,
@@ -64,11 +80,10 @@ __global__ __launch_bounds__(kPoolMaxThreads<ROPE>) void pool_kernel(PoolParams 
     }
     const int c0 = p.heads[0] * 8, c1 = p.heads[1] * 8, c2 = p.heads[2] * 8;
     const int ctot = c0 + c1 + c2;
-    constexpr int TPC = kThreadsPerChunk<ROPE>;
-    const int hb = TPC == 2 ? (p.bs + 1) >> 1 : p.bs;  // tokens of the first (or only) half
-    // blockDim.x is even, so the two threads of a column are adjacent lanes of one iteration
-    for (int col2 = threadIdx.x; col2 < TPC * ctot; col2 += blockDim.x) {
-        const int col = TPC == 2 ? col2 >> 1 : col2, half = TPC == 2 ? col2 & 1 : 0;
+    // whole waves (blockDim.x is a multiple of 64): the threads of a chunk are adjacent lanes of
+    // one iteration
+    for (int item = threadIdx.x + blockIdx.z * blockDim.x; item < TPC * ctot; item += blockDim.x * gridDim.z) {
+        const int col = item / TPC, part = item % TPC;
         const int which = col < c0 ? 0 : (col < c0 + c1 ? 1 : 2);
         const int cc = col - (which == 0 ? 0 : (which == 1 ? c0 : c0 + c1));
         const int hd = cc >> 3, ch = cc & 7;
@@ -94,14 +109,14 @@ __global__ __launch_bounds__(kPoolMaxThreads<ROPE>) void pool_kernel(PoolParams 
             }
         };
         if (t >= p.nb) {  // padding blocks of the operand-ordered outputs
-            if (frag && half == 0) {
+            if (frag && part == 0) {
                 const float zero[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
                 store_frag(zero);
             }
             continue;
         }
-        // tokens n0 .. n1-1 of the block: this thread's half
-        const int n0 = half ? hb : 0, n1 = half ? p.bs : hb;
+        // tokens n0 .. n1-1 of the block: this thread's run
+        const int n0 = part * p.bs / TPC, n1 = (part + 1) * p.bs / TPC;
         const int64_t sn = sel3(p.sn, which);
         const int64_t tok0 = (int64_t)t * p.bs + n0;
         const bf16_t* src = sel3(p.x, which) + b * sel3(p.sb, which) + tok0 * sn + (int64_t)hd * sel3(p.sh, which) + ch * 8;
@@ -171,21 +186,18 @@ __global__ __launch_bounds__(kPoolMaxThreads<ROPE>) void pool_kernel(PoolParams 
             }
             add_token(v);
         }
-        // first half + second half, the same sum in both lanes of the pair (a one-token block
-        // has no second half: its sum is kept as is)
-        if (p.bs > hb) {
+        // the block's sum and maximum in every thread of the chunk (an empty run adds 0)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) acc[e] = acc_pair(acc[e], half);
-            sqmax = fmaxf(sqmax, swap_pair(sqmax));
-        }
-        if (which == 1 && p.kbnd != nullptr && half == 0)
+        for (int e = 0; e < 8; ++e) acc[e] = chunk_add<TPC>(acc[e]);
+        sqmax = chunk_max<TPC>(sqmax);
+        if (which == 1 && p.kbnd != nullptr && part == 0)
             p.kbnd[(((int64_t)b * p.nb + t) * heads + hd) * 8 + ch] = sqmax;
         const float denom = (float)p.bs;
         float mean[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) mean[e] = acc[e] / denom;
         bf16_t* out = sel3(p.out_bnhd, which);
-        if (out && half == 0) {
+        if (out && part == 0) {
             uint4 w;
             w.x = pack_bf16x2(mean[0], mean[1]);
             w.y = pack_bf16x2(mean[2], mean[3]);
@@ -193,7 +205,39 @@ __global__ __launch_bounds__(kPoolMaxThreads<ROPE>) void pool_kernel(PoolParams 
             w.w = pack_bf16x2(mean[6], mean[7]);
             *reinterpret_cast<uint4*>(out + (((int64_t)b * p.nb + t) * heads + hd) * kHeadDim + ch * 8) = w;
         }
-        if (frag && half == (p.bs > hb ? 1 : 0)) store_frag(mean);  // both halves hold the mean
+        if (frag && part == TPC - 1) store_frag(mean);  // every part holds the mean
+    }
+}
+
+// Threads per column chunk and per workgroup (0: one workgroup for all columns of a block).
+// One thread per chunk (two with RoPE, whose rotation doubles the arithmetic) is the fastest
+// while the blocks alone keep the chip busy; below that the pass is one serial walk of the
+// block per thread, so the walk is split, to runs of eight tokens (one round of loads) at the
+// shortest, until about one wave per SIMD is in flight (three with RoPE), and a block's columns
+// go to workgroups of their own.  Pass alone, 1 thread -> the split: Nside 16, 20/5 heads 6.7 ->
+// 4.9 us (180 -> 1440 waves), Nside 32, 12/3 heads 7.5 -> 5.8 us, 16/4 heads with 128-token
+// blocks 13.4 -> 8.4 us, that shape's keys alone 11.7 -> 4.1 us; with RoPE the whole op there
+// 118 -> 109 us.  At Nside 64 splitting only adds the sums' exchange (18.6 -> 19.3 us at four
+// threads).  The largest passes (24 members) stream from HBM and gain from two threads and
+// smaller workgroups again: 176 -> 167 us (8 members: 48.4 -> 51.3 us, so not there).
+struct PoolShape { int tpc, wg; };
+PoolShape pool_shape(const PoolParams& p, int chunks) {
+    const int64_t waves = (int64_t)chunks * p.nb * p.B / 64;  // at one thread per chunk
+    if (waves >= 8192) return {2, 256};
+    const bool rope = p.rope_cos != nullptr;
+    int tpc = rope ? 2 : 1;
+    const int first = tpc;
+    while (tpc < 8 && waves * tpc < (rope ? 3072 : 768) && p.bs >= 16 * tpc) tpc *= 2;
+    return {tpc, tpc > first ? (rope ? 256 : 128) : 0};
+}
+
+template <int ROPE>
+const void* pool_fn(int tpc) {
+    switch (tpc) {
+        case 1: return (const void*)pool_kernel<ROPE, 1>;
+        case 2: return (const void*)pool_kernel<ROPE, 2>;
+        case 4: return (const void*)pool_kernel<ROPE, 4>;
+        default: return (const void*)pool_kernel<ROPE, 8>;
     }
 }
 
@@ -206,13 +250,15 @@ hipError_t launch_pool(const PoolParams& p, hipStream_t s) {
     void* args[] = {&q};
     const int tgrid = (p.kfrag || p.vfrag) ? p.nb_pad : p.nb;
     const size_t lds = q.rope_lds ? (size_t)p.bs * 256 : 0;
-    const void* fn = p.rope_cos == nullptr ? (const void*)pool_kernel<0>
-                   : q.rope_lds ? (const void*)pool_kernel<1> : (const void*)pool_kernel<2>;
-    // one thread (two with RoPE) per 16-byte column chunk of the q, k, v rows, in whole waves
-    const int items = (p.rope_cos != nullptr ? 2 : 1) * 8 * (p.heads[0] + p.heads[1] + p.heads[2]);
+    const int chunks = 8 * (p.heads[0] + p.heads[1] + p.heads[2]);
+    const PoolShape shape = pool_shape(p, chunks);
+    const void* fn = p.rope_cos == nullptr ? pool_fn<0>(shape.tpc) : q.rope_lds ? pool_fn<1>(shape.tpc) : pool_fn<2>(shape.tpc);
+    // tpc threads per 16-byte column chunk of the q, k, v rows, in whole waves
+    const int items = shape.tpc * chunks;
     const int cap = p.rope_cos == nullptr ? kPoolMaxThreads<0> : q.rope_lds ? kPoolMaxThreads<1> : kPoolMaxThreads<2>;
-    const int threads = items >= cap ? cap : (items + 63) / 64 * 64;
-    return hipLaunchKernel(fn, dim3(tgrid, p.B), dim3(threads), args, lds, s);
+    const int threads = std::min((items + 63) / 64 * 64, shape.wg > 0 ? shape.wg : cap);
+    const int z = shape.wg > 0 ? (items + threads - 1) / threads : 1;
+    return hipLaunchKernel(fn, dim3(tgrid, p.B, z), dim3(threads), args, lds, s);
 }
 
 }  // namespace mosaic

@@ -470,3 +470,20 @@ def test_mosaic_attention_module_runs():
         assert y.shape == x.shape and torch.isfinite(y.float()).all()
         m._shared_rope_tables = lambda: False
         assert torch.equal(m(x), y)   # RoPE modules, then the op
+
+
+@pytest.mark.parametrize("B,N,H,bs", [
+    (1, 192, 1, 64), (1, 3072, 5, 64), (2, 1536, 3, 128), (1, 2048, 2, 1024), (1, 600, 3, 24), (1, 1400, 7, 200),
+    (1, 24576, 12, 64), (1, 49152, 18, 64), (12, 49152, 16, 64)],
+    ids=["one_head", "small", "bs128", "bs1024", "bs24", "bs200", "four_threads", "one_thread", "largest"])
+def test_pool_mean_thread_splits(B, N, H, bs):
+    """Every split of a block's token walk (1, 2, 4 and 8 threads per column chunk; runs of
+    unequal length at 24 and 200 tokens): within half a bf16 spacing (2^-8 relative) of the
+    float64 mean, plus the fp32 sum's bound bs 2^-24 mean|x|."""
+    print(f"pool split B={B} N={N} H={H} bs={bs}", flush=True)
+    x = torch.randn(B, N, H, 64, generator=torch.Generator(DEV).manual_seed(N + bs), device=DEV).to(torch.bfloat16)
+    got = M.pool_mean(x, bs)
+    blocks = x.view(B, N // bs, bs, H, 64)
+    ref = blocks.mean(2, dtype=torch.float64)
+    bound = 2 ** -8 * ref.abs() + bs * 2 ** -24 * blocks.abs().mean(2, dtype=torch.float64)
+    assert got.shape == ref.shape and ((got.double() - ref).abs() <= bound).all()
