@@ -22,7 +22,7 @@
 extern "C" {
 #endif
 
-#define MOSAIC_BSA_ABI_VERSION 10
+#define MOSAIC_BSA_ABI_VERSION 11
 
 #if defined(__GNUC__) || defined(__clang__)
 #define MOSAIC_API __attribute__((visibility("default")))
@@ -425,6 +425,13 @@ MOSAIC_API int mosaic_swiglu_fwd(const void* h, int32_t dtype, int64_t rows, int
 MOSAIC_API int mosaic_swiglu_linear_fwd(const void* x, int64_t rows, int32_t dim, int64_t x_row_stride,
                                         const void* weight, int32_t hidden, const void* noise,
                                         int32_t noise_rows, void* out, void* stream);
+
+/* mosaic_swiglu_linear_fwd on w13 as the Linear stores it (bf16 [2*hidden, dim] contiguous, the
+   x1 half's rows, then the x3 half's), for any rows >= 256; the other arguments, limits and the
+   result as there. */
+MOSAIC_API int mosaic_swiglu_linear_w13_fwd(const void* x, int64_t rows, int32_t dim, int64_t x_row_stride,
+                                            const void* w13, int32_t hidden, const void* noise,
+                                            int32_t noise_rows, void* out, void* stream);
 
 /* Name of a status code (static storage). */
 MOSAIC_API const char* mosaic_bsa_strerror(int status);

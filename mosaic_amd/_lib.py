@@ -12,7 +12,7 @@ import threading
 
 LIB_NAME = "libmosaic_bsa.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 # mosaic_bsa_mode
 MODE_FULL = 0
@@ -57,6 +57,7 @@ EXPORTED_SYMBOLS = (
     "mosaic_gate_softmax_fwd",
     "mosaic_add_merge_fwd",
     "mosaic_swiglu_linear_fwd",
+    "mosaic_swiglu_linear_w13_fwd",
     "mosaic_sparse_attn_fwd",
     "mosaic_sparse_attn_fwd_workspace_size",
     "mosaic_sparse_attn_fwd_ws",
@@ -154,6 +155,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.mosaic_add_merge_fwd.restype = c_int
     lib.mosaic_swiglu_linear_fwd.argtypes = [c_vp, c_i64, c_i32, c_i64, c_vp, c_i32, c_vp, c_i32, c_vp, c_vp]
     lib.mosaic_swiglu_linear_fwd.restype = c_int
+    lib.mosaic_swiglu_linear_w13_fwd.argtypes = lib.mosaic_swiglu_linear_fwd.argtypes
+    lib.mosaic_swiglu_linear_w13_fwd.restype = c_int
     lib.mosaic_sparse_attn_bwd_workspace_size.argtypes = [c_i32, c_i32, c_i32]
     lib.mosaic_sparse_attn_bwd_workspace_size.restype = c_size
     lib.mosaic_sparse_attn_bwd.argtypes = [Bnhd, Bnhd, Bnhd, c_vp, c_vp, Bnhd, c_vp, c_i32, c_i32, c_i32, c_i32,

@@ -15,6 +15,7 @@
   RMSNorm in one pass.
 * ``swiglu_linear(x, w13_perm, noise)``: cSwiGLU's ``w13`` projection and that gate in one
   kernel (h is never stored); ``permute_w13`` lays out the weight it takes.
+  ``swiglu_linear_w13(x, w13, noise)`` is the same on the weight as the Linear stores it.
 
 Inputs must be on a ROCm device; there is no CPU path.  ``autocast_dtype`` reports the dtype
 torch's own RMSNorm returns under the current autocast state, so the fused norm's output has
@@ -29,7 +30,7 @@ import torch.nn as nn
 from . import _lib
 from .ops import forward_only, stream_of
 
-__all__ = ["RMSNorm", "rms_norm", "swiglu", "swiglu_linear", "permute_w13", "swiglu_linear_ok", "autocast_dtype",
+__all__ = ["RMSNorm", "rms_norm", "swiglu", "swiglu_linear", "swiglu_linear_w13", "permute_w13", "swiglu_linear_ok", "autocast_dtype",
            "resample_norm", "gate_softmax", "add_merge"]
 
 _DT = {torch.float32: _lib.DTYPE_F32, torch.bfloat16: _lib.DTYPE_BF16}
@@ -183,6 +184,44 @@ def swiglu_linear(x: torch.Tensor, w13_perm: torch.Tensor, noise: torch.Tensor |
                                              n.data_ptr() if n is not None else None,
                                              n.shape[0] if n is not None else 0, out.data_ptr(), stream_of(x))
     _lib.check(st, "mosaic_swiglu_linear_fwd")
+    return out
+
+
+def swiglu_linear_pays(rows: int, hidden: int) -> bool:
+    """Whether w13 and the gate are faster as one kernel than as the library GEMM and the gate
+    kernel: with enough of its 256-row x 128-index tiles for a quarter of the compute units.
+    Measured one against two, us: 768 rows of dim 768 (72 tiles) 20.8 / 21.0, 1024 rows 21.4 /
+    23.9, of dim 512 (64 tiles) 16.8 / 16.9, of dim 256 (32 tiles) 12.5 / 10.5, 512 rows of dim
+    1280 (80 tiles) 28.7 / 25.7; from 1536 rows on 1.2 to 2.3 times faster throughout."""
+    return rows >= 1024 and -(-rows // 256) * (hidden // 128) >= 64
+
+
+def swiglu_linear_w13_ok(x: torch.Tensor, w13: torch.Tensor, noise: torch.Tensor | None) -> bool:
+    """Whether ``swiglu_linear_w13`` takes these: contiguous, 16-byte aligned bf16 tensors on one
+    ROCm device, at least 256 rows, dim and hidden multiples of 128, one noise row per member."""
+    two_h, dim = w13.shape
+    ts = (x, w13) if noise is None else (x, w13, noise)
+    return (all(t.is_cuda and t.dtype == torch.bfloat16 and t.device == x.device and t.is_contiguous()
+                and t.data_ptr() % 16 == 0 for t in ts)
+            and x.dim() >= 2 and x.shape[-1] == dim and x.numel() >= 256 * dim and dim % 128 == 0 and two_h % 256 == 0
+            and (noise is None or tuple(noise.shape) == (x.shape[-2], two_h // 2)))
+
+
+def swiglu_linear_w13(x: torch.Tensor, w13: torch.Tensor, noise: torch.Tensor | None = None) -> torch.Tensor:
+    """``swiglu(x @ w13^T, noise)`` in one kernel, w13 bf16 ``[2*hidden, dim]`` as the Linear
+    stores it.  x: bf16 ``[..., dim]`` (``[S, B, dim]`` when noise ``[B, hidden]`` is given), 256
+    rows or more.  Rounding points as ``swiglu_linear``.  Returns ``[..., hidden]``."""
+    forward_only("fused.swiglu_linear_w13", x, w13, noise)
+    if not swiglu_linear_w13_ok(x, w13, noise):
+        raise ValueError("swiglu_linear_w13 needs contiguous bf16 ROCm tensors of 256 rows or more, dim % 128 == 0, "
+                         "hidden % 128 == 0 and one noise row per member")
+    two_h, dim = w13.shape
+    out = torch.empty(*x.shape[:-1], two_h // 2, dtype=torch.bfloat16, device=x.device)
+    st = _lib.lib().mosaic_swiglu_linear_w13_fwd(x.data_ptr(), x.numel() // dim, dim, dim, w13.data_ptr(), two_h // 2,
+                                                 noise.data_ptr() if noise is not None else None,
+                                                 noise.shape[0] if noise is not None else 0, out.data_ptr(),
+                                                 stream_of(x))
+    _lib.check(st, "mosaic_swiglu_linear_w13_fwd")
     return out
 
 

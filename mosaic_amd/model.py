@@ -6,8 +6,9 @@ building blocks of primitives.py it composes (``MosaicBlock``, ``cSwiGLU``,
 and parameter names, so a reference state dict loads unchanged.  Every attention layer runs
 ``MosaicAttention`` (the op in libmosaic_bsa.so, RoPE fused into its pooling pass) and both
 grid interpolations run ``CrossAttentionInterpolate`` (the k-NN gather-attention kernel).  The
-projections are library GEMMs; the RMSNorms and the SwiGLU gate run as the fused HIP kernels of
-``mosaic_amd.fused`` when their inputs are on a ROCm device.
+projections are library GEMMs except the feed-forward's w13, which runs with its gate as one HIP
+kernel; that one and the RMSNorms are the fused kernels of ``mosaic_amd.fused``, used when their
+inputs are on a ROCm device.
 
 Activations are sequence-first ``[S, B, C]`` (S pixels, B = members x noise samples), as in
 the reference.  The model runs under ``torch.autocast('cuda', torch.bfloat16)``.  The
@@ -145,28 +146,37 @@ class cSwiGLU(nn.Module):
         if noise_dim > 0:
             self.noise_bias = nn.Linear(noise_dim, hidden_dim, bias=False)
 
-    # With this set (and on a ROCm device with bf16 input of qualifying shape), w13 and the gate
-    # run as one kernel (fused.swiglu_linear) on a row-permuted bf16 copy of w13, so h is never
-    # stored.  Off by default: at the era5 stage-1 shape (1,179,648 rows, 768 -> 2 x 3072, 24
-    # members) the fused kernel takes 15.3 ms against 14.1 ms for the library GEMM (9.4 ms)
-    # followed by the gate kernel; its GEMM core alone (epilogue arithmetic removed) takes
-    # 12.8 ms, slower than the library's.
-    fused_linear_gate = False
+    # Whether w13 and the gate run as one kernel (fused.swiglu_linear_w13: h is never stored) where
+    # it computes what w13 under the current autocast state and the gate kernel would: 9.3 against
+    # 13.8 ms at the era5 stage-1 shape with 24 members (1,179,648 rows, 768 -> 2 x 3072), 0.40
+    # against 0.60 ms with one.
+    fused_linear_gate = True
 
-    def _w13_perm(self) -> torch.Tensor:
-        wt = self.w13.weight
-        key = (wt.data_ptr(), wt._version, wt.device, wt.dtype)
-        if getattr(self, "_w13_perm_key", None) != key:
-            with torch.no_grad():
-                self._w13_perm_cache = fused.permute_w13(wt.detach().to(torch.bfloat16))
-            self._w13_perm_key = key
-        return self._w13_perm_cache
+    def _one_kernel(self, x: torch.Tensor, noise: torch.Tensor | None) -> torch.Tensor | None:
+        """w13 and the gate as one kernel, or None where they run as two: w13 replaced, hooked or
+        biased, arithmetic other than bf16, or a shape the kernel does not take."""
+        lin = self.w13
+        if (type(lin) is not nn.Linear or type(lin.weight) is not nn.Parameter or lin.bias is not None
+                or type(x) is not torch.Tensor or not x.is_cuda or x.dtype != torch.bfloat16
+                or lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks or lin._backward_pre_hooks
+                or torch.nn.modules.module._has_any_global_hook()):
+            return None
+        forward_only("cSwiGLU", x, lin.weight, noise)
+        if torch.is_autocast_enabled("cuda"):
+            if torch.get_autocast_dtype("cuda") != torch.bfloat16:
+                return None
+        elif lin.weight.dtype != torch.bfloat16:
+            return None
+        if x.dim() < 2 or not fused.swiglu_linear_pays(x.numel() // max(1, x.shape[-1]), lin.out_features // 2):
+            return None
+        w = lin.weight.to(torch.bfloat16)
+        return fused.swiglu_linear_w13(x, w, noise) if fused.swiglu_linear_w13_ok(x, w, noise) else None
 
     def forward(self, x: torch.Tensor, z: torch.Tensor | None = None) -> torch.Tensor:
         noise = self.noise_bias(z) if z is not None else None      # [B, hidden]
-        if self.fused_linear_gate and fused.swiglu_linear_ok(x, self.w2.in_features):
-            forward_only("cSwiGLU", x, self.w13.weight, noise)
-            return self.w2(fused.swiglu_linear(x, self._w13_perm(), noise))
+        g = self._one_kernel(x, noise) if self.fused_linear_gate else None
+        if g is not None:
+            return self.w2(g)
         h = self.w13(x)
         if h.is_cuda:
             g = fused.swiglu(h, noise)

@@ -98,3 +98,84 @@ def test_cswiglu_refuses_grad(fused_gate):
     x = torch.randn(256, 1, 256, device=DEV, dtype=torch.bfloat16)
     with pytest.raises(RuntimeError, match="no backward"):
         m(x)
+
+
+@pytest.mark.parametrize("S,B,dim,hidden,noise", [
+    (256, 1, 128, 128, True),       # one tile, the shortest reduction
+    (257, 1, 256, 128, True),       # a last row tile that starts one row after the first
+    (1000, 3, 384, 256, True),      # ragged rows, members that do not divide a tile
+    (19, 56, 256, 384, True),       # the most noise rows staged in LDS
+    (18, 57, 256, 384, True),       # one more: noise from global memory
+    (4100, 1, 1280, 640, False),    # 85 tiles in a partial last round over the XCDs, no noise
+    (2048, 2, 128, 1280, True),     # several tiles per workgroup with two iterations each
+])
+def test_swiglu_linear_w13_shapes(S, B, dim, hidden, noise):
+    """The kernel on w13 as stored, at the edges of its tiles, noise paths and tile rounds, on a
+    poisoned allocation: every row written, against the fp32-accumulate reference."""
+    print(f"swiglu_linear_w13 S={S} B={B} dim={dim} hidden={hidden} noise={noise}", flush=True)
+    g = torch.Generator().manual_seed(S + B + dim)
+    x = torch.randn(S, B, dim, generator=g).to(torch.bfloat16)
+    w13 = (torch.randn(2 * hidden, dim, generator=g) * dim ** -0.5).to(torch.bfloat16)
+    nz = torch.randn(B, hidden, generator=g).to(torch.bfloat16) if noise else None
+    torch.full((S, B, hidden), float("nan"), dtype=torch.bfloat16, device=DEV)   # freed: the next output's memory
+    with torch.no_grad():
+        got = fused.swiglu_linear_w13(x.to(DEV), w13.to(DEV), nz.to(DEV) if noise else None)
+    ref = reference(x, w13, nz)
+    check(got, ref, "vs fp32-accumulate reference")
+    # only sums in another order and the silu's last fp32 bits differ: bf16 roundings rarely flip
+    assert (got.cpu() == ref).float().mean().item() >= 0.999
+
+
+def test_swiglu_linear_w13_non_finite_rows_stay_in_their_rows():
+    x = torch.randn(600, 1, 256, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16)
+    w13 = (torch.randn(512, 256, generator=torch.Generator().manual_seed(4)) / 16).to(torch.bfloat16)
+    clean = fused.swiglu_linear_w13(x.to(DEV), w13.to(DEV)).cpu()
+    x[5, 0, 7], x[599, 0, 0] = float("inf"), float("nan")
+    got = fused.swiglu_linear_w13(x.to(DEV), w13.to(DEV)).cpu()
+    keep = torch.ones(600, dtype=torch.bool)
+    keep[[5, 599]] = False
+    assert torch.equal(got[keep], clean[keep]) and got[599].isnan().all()
+    want = fused.swiglu((x[5:6].to(DEV) @ w13.to(DEV).t())).cpu()
+    assert torch.equal(got[5].isnan(), want[0].isnan()) and torch.equal(got[5].isinf(), want[0].isinf())
+
+
+@pytest.mark.parametrize("change", ["none", "hook", "global_hook", "bias", "replaced", "fp32_noise", "odd_rows", "view"])
+def test_cswiglu_routes(change, monkeypatch):
+    """The module takes the one kernel only where nothing observes or replaces w13 and the shape
+    fits, and its result is the two-step one on every route."""
+    torch.manual_seed(1)
+    m = cSwiGLU(256, 1024, 64).to(DEV)
+    x = torch.randn(1030, 2, 256, device=DEV).to(torch.bfloat16)
+    z = torch.randn(2, 64, device=DEV)
+    calls, seen = [], []
+    real = fused.swiglu_linear_w13
+    monkeypatch.setattr(fused, "swiglu_linear_w13", lambda *a: calls.append(1) or real(*a))
+    handle = None
+    if change == "hook":
+        m.w13.register_forward_hook(lambda *a: seen.append(1))
+    elif change == "global_hook":
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda mod, *a: seen.append(1) if mod is m.w13 else None)
+    elif change == "bias":
+        lin = torch.nn.Linear(256, 2048).to(DEV)
+        lin.weight = m.w13.weight
+        m.w13 = lin
+    elif change == "replaced":
+        m.w13 = torch.nn.Sequential(m.w13)
+    elif change == "fp32_noise":
+        m.noise_bias = torch.nn.Identity()
+        z = torch.randn(2, 1024, device=DEV)
+    elif change == "odd_rows":
+        x = x[:100]
+    elif change == "view":
+        x = torch.randn(1030, 2, 512, device=DEV).to(torch.bfloat16)[..., 128:384]
+    try:
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+            got = m(x, z)
+            n, m.fused_linear_gate = len(calls), False
+            want = m(x, z)
+    finally:
+        if handle is not None:
+            handle.remove()
+    assert n == (1 if change == "none" else 0) and len(calls) == n
+    assert len(seen) == (2 if "hook" in change else 0)
+    check(got, want, change)
