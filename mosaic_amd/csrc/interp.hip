@@ -11,22 +11,24 @@
 // to_q, and the k / v rows are read straight from [S_from, B, H, 64] (neighbouring targets
 // share most of their neighbours, so rows are reused from L2).
 //
-// The work is VALU-bound: every (target, member, head) takes 2 K 64 bf16-rounded products.
-// Each product is one v_dot2_f32_bf16 of the packed k / v pair against (x, 0) or (0, x)
-// (exact: a bf16 x bf16 product fits fp32), then half a v_cvt_pk_bf16_f32 and half a
-// v_dot2_f32_bf16 that adds the rounded pair; no k / v element is unpacked to fp32.
-// Staging each tile of targets' neighbour union in LDS (cutting the L2 requests 4-7x)
-// measured slower than this direct form: it halves the occupancy, and occupancy is what
-// hides the latency of the reduction chains.
+// Two forms of the two weighted sums: products rounded to bf16 before they are added (the
+// reference's eager elementwise ops) and exact products summed in fp32 (its compiled path).
 //
-// One wave per (target s, head h) pair, looping over the batch members b with the next
-// member's k / v loaded as soon as the current member is done with them.  Lane l = 8 jg + dc holds the 8-dim chunk dc of neighbours
-// jg + 8 i (its "slots"): every k / v read is a 16-byte load and each 128-byte row is read
-// by 8 adjacent lanes.  Scores are summed over the 8 chunk lanes with DPP (lanes l ^ 1,
-// l ^ 2, l ^ 4), the softmax max / sum over the 8 neighbour groups with DPP row_ror:8,
-// v_permlane16_swap and v_permlane32_swap; the output's 8 partial sums per lane are
-// reduce-scattered over the groups by the same three exchanges, leaving one dimension per
-// lane.  Workgroups are remapped so that each XCD takes one contiguous range of targets, in
+// The bf16-product form is VALU-bound: every (target, member, head) takes 2 K 64 rounded
+// products.  Each product is one v_dot2_f32_bf16 of the packed k / v pair against (x, 0) or
+// (0, x) (exact: a bf16 x bf16 product fits fp32), then half a v_cvt_pk_bf16_f32 and half a
+// v_dot2_f32_bf16 that adds the rounded pair; no k / v element is unpacked to fp32.
+//
+// Per-target kernel: one wave per (target s, head h) pair, looping over the batch members b with
+// the next member's k / v loaded as soon as the current member is done with them.  Lane l = 8
+// jg + dc holds the 8-dim chunk dc of neighbours jg + 8 i (its "slots"): every k / v read is a
+// 16-byte load and each 128-byte row is read by 8 adjacent lanes.  Scores are summed over the 8
+// chunk lanes with DPP, the softmax max / sum over the 8 neighbour groups with DPP row_ror:8,
+// v_permlane16_swap and v_permlane32_swap.  The output of the bf16-product form: the 8 partial
+// sums per lane are reduce-scattered over the groups by the same three exchanges, leaving one
+// dimension per lane; of the fp32 form: v and the weights go through LDS (weighted_sum).
+// The fp32 form also has an LDS-staged kernel, for tiles of targets (below).
+// Workgroups are remapped so that each XCD takes one contiguous range of targets, in
 // the caller's target order when one is given: with targets sorted along a space-filling
 // curve, the waves in flight on an XCD share most of their neighbours' rows in its L2.
 #include "bsa_common.h"
@@ -58,6 +60,13 @@ __device__ __forceinline__ float chunk_sum(float x) {
     x = dpp_add<0xb1>(x);      // quad_perm [1,0,3,2]
     x = dpp_add<0x4e>(x);      // quad_perm [2,3,0,1]
     return dpp_add<0x141>(x);  // row_half_mirror
+}
+
+// the same sum in the order of the fp32-product form: lane 7 - l of the group, then l ^ 2, l ^ 1
+__device__ __forceinline__ float dot_chunk_sum(float x) {
+    x = dpp_add<0x141>(x);
+    x = dpp_add<0x4e>(x);
+    return dpp_add<0xb1>(x);
 }
 
 // v_permlane16_swap(a, b): rows 1 and 3 of a trade places with rows 0 and 2 of b.  The
@@ -243,18 +252,6 @@ __device__ __forceinline__ float score_dot(const uint32_t (&q)[4], const uint4& 
     a = __builtin_amdgcn_fdot2_f32_bf16(as_bf2(q[2]), as_bf2(k.z), a, false);
     return __builtin_amdgcn_fdot2_f32_bf16(as_bf2(q[3]), as_bf2(k.w), a, false);
 }
-// One neighbour (weight w as (w, 0) and (0, w)) against the lane's eight output dimensions in
-// fp32: acc[d] (+)= w v[d], one dot product per product.
-template <bool FIRST>
-__device__ __forceinline__ void out_fp32(uint32_t w_lo, uint32_t w_hi, const uint4& v, float* acc) {
-    const uint32_t vv[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        acc[2 * e] = __builtin_amdgcn_fdot2_f32_bf16(as_bf2(w_lo), as_bf2(vv[e]), FIRST ? 0.f : acc[2 * e], false);
-        acc[2 * e + 1] = __builtin_amdgcn_fdot2_f32_bf16(as_bf2(w_hi), as_bf2(vv[e]), FIRST ? 0.f : acc[2 * e + 1], false);
-    }
-}
-
 // The score of a slot in base-2 units, sc = bf16(bf16(part) * scale) * log2 e.  A power-of-two
 // scale leaves bf16(part) * scale a bf16 value (a product too small to be normal is below
 // 2^-126 in magnitude, and so is the difference its rounding would make), so that case takes
@@ -281,29 +278,94 @@ __device__ __forceinline__ void softmax_weights(const float (&sc)[NSLOT], float 
     for (int i = 0; i < NSLOT; ++i) w[i] *= inv;
 }
 
-// acc[d] = sum over the lane's slots of w * v[d] with exact products, slot by slot
+// The order of the neighbours in the fp32-product output sum: position pos of 8 NSLOT holds
+// neighbour knn_order(pos).  Slots 2m and 2m + 1 alternate, so the weights of a neighbour group
+// (jg) form one packed pair; an odd last slot follows in its own order.
 template <int NSLOT>
-__device__ __forceinline__ void weighted_sum_fp32(const float (&w)[NSLOT], const uint4 (&vw)[NSLOT], float (&acc)[8]) {
+__device__ __forceinline__ constexpr int knn_order(int pos) {
+    return pos < 16 * (NSLOT / 2) ? 16 * (pos / 16) + 8 * (pos & 1) + (pos % 16) / 2 : pos;
+}
+// This lane's weights (slots w[i], neighbours jg + 8 i) into a target's weight table at lds:
+// bf16, in the order of knn_order.
+template <int NSLOT>
+__device__ __forceinline__ void put_weights(const float (&w)[NSLOT], char* lds, int jg) {
+#pragma unroll
+    for (int i = 0; i + 1 < NSLOT; i += 2) *reinterpret_cast<uint32_t*>(lds + 16 * i + 4 * jg) = pack_bf16x2(w[i], w[i + 1]);
+    if constexpr (NSLOT & 1)
+        *reinterpret_cast<uint16_t*>(lds + 16 * (NSLOT - 1) + 2 * jg) = (uint16_t)(pack_bf16x2(w[NSLOT - 1], 0.f) & 0xffffu);
+}
+// Four neighbours' values of dimension d = lane: a transposing read, in which lane l addresses
+// dimensions 16 (l / 16) + 4 (l % 4) .. + 3 of the row of position (l / 4) % 4.
+typedef short v4i16_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint2 read_v4(uint32_t lds, int offset = 0) {
+    auto* const a = (__attribute__((address_space(3))) char*)(uintptr_t)lds + offset;
+    return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16_t*)a));
+}
+// Output dimension d = lane of one target, fp32 products: v_mfma_f32_4x4x4_16b_bf16 multiplies,
+// in each block of four lanes, four neighbours' values of the lanes' dimensions (vv) with rows
+// of weights; every lane holds the same weights (ww), so every row of the result is the output.
+// One instruction takes four neighbours, in position order, accumulating in fp32.
+template <int NSLOT>
+__device__ __forceinline__ float weighted_sum(const uint4 (&ww)[NSLOT], const uint2 (&vv)[2 * NSLOT]) {
+    f32x4 a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < NSLOT; ++i) {
-        const uint32_t w_lo = pack_bf16x2(w[i], 0.f), w_hi = pack_bf16x2(0.f, w[i]);
-        if (i == 0) out_fp32<true>(w_lo, w_hi, vw[i], acc);
-        else out_fp32<false>(w_lo, w_hi, vw[i], acc);
+        a = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(v4i16_t, make_uint2(ww[i].x, ww[i].y)),
+                                                   __builtin_bit_cast(v4i16_t, vv[2 * i]), a, 0, 0, 0);
+        a = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(v4i16_t, make_uint2(ww[i].z, ww[i].w)),
+                                                   __builtin_bit_cast(v4i16_t, vv[2 * i + 1]), a, 0, 0, 0);
     }
+    return a[0];
 }
 
-// The lane's 8 partial output dimensions reduce-scattered over the 8 neighbour groups: halves
-// (dims e / e + 4), row pairs (e / e + 2), then lanes l ^ 8 (e / e + 1); the lane ends up with
-// dimension 8 dc + 4 (l / 32) + 2 ((l / 16) % 2) + (l / 8) % 2 summed over all neighbours.
-__device__ __forceinline__ float reduce_scatter(const float (&acc)[8], int lane) {
-    float r4[4], r2[2];
+// The to_q rows of a lane's eight dimensions (three bf16 weights each: 48 bytes, 16-byte
+// aligned) as packed (w0, w1) and (w2, 0), and eight query values bf16(rel . w) from a
+// neighbour's rel = (r0, r1), (r2, 0), as packed pairs: fp32 sums of the exact products.
+struct QueryRows { uint32_t w01[8], w2[8]; };
+__device__ __forceinline__ QueryRows query_rows(const bf16_t* wr) {
+    uint32_t u[12];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) r4[e] = swap32_add(acc[e], acc[e + 4]);
+    for (int c = 0; c < 3; ++c) {
+        const uint4 x = ld16(wr + 8 * c);
+        u[4 * c] = x.x; u[4 * c + 1] = x.y; u[4 * c + 2] = x.z; u[4 * c + 3] = x.w;
+    }
+    QueryRows r;
 #pragma unroll
-    for (int e = 0; e < 2; ++e) r2[e] = swap16_add(r4[e], r4[e + 2]);
-    const bool odd8 = lane & 8;
-    const float keep = odd8 ? r2[1] : r2[0], give = odd8 ? r2[0] : r2[1];
-    return keep + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(give), 0x128, 0xf, 0xf, false));
+    for (int e = 0; e < 8; e += 2) {
+        const uint32_t* t = u + 3 * (e / 2);  // w0 w1 | w2 w0' | w1' w2'
+        r.w01[e] = t[0];
+        r.w2[e] = t[1] & 0xffffu;
+        r.w01[e + 1] = (t[1] >> 16) | (t[2] << 16);
+        r.w2[e + 1] = t[2] >> 16;
+    }
+    return r;
+}
+__device__ __forceinline__ void query_pairs(const QueryRows& w, uint32_t r01, uint32_t r2, uint32_t (&q)[4]) {
+    float a0, a1, a2, a3, a4, a5, a6, a7;
+    // the eight first products from a literal 0 addend, the second ones through the
+    // accumulator (no wait between them), then the three wait states before the conversions
+    asm("v_dot2_f32_bf16 %0, %8, %10, 0\n\t"
+        "v_dot2_f32_bf16 %1, %8, %11, 0\n\t"
+        "v_dot2_f32_bf16 %2, %8, %12, 0\n\t"
+        "v_dot2_f32_bf16 %3, %8, %13, 0\n\t"
+        "v_dot2_f32_bf16 %4, %8, %14, 0\n\t"
+        "v_dot2_f32_bf16 %5, %8, %15, 0\n\t"
+        "v_dot2_f32_bf16 %6, %8, %16, 0\n\t"
+        "v_dot2_f32_bf16 %7, %8, %17, 0\n\t"
+        "v_dot2_f32_bf16 %0, %9, %18, %0\n\t"
+        "v_dot2_f32_bf16 %1, %9, %19, %1\n\t"
+        "v_dot2_f32_bf16 %2, %9, %20, %2\n\t"
+        "v_dot2_f32_bf16 %3, %9, %21, %3\n\t"
+        "v_dot2_f32_bf16 %4, %9, %22, %4\n\t"
+        "v_dot2_f32_bf16 %5, %9, %23, %5\n\t"
+        "v_dot2_f32_bf16 %6, %9, %24, %6\n\t"
+        "v_dot2_f32_bf16 %7, %9, %25, %7\n\t"
+        "s_nop 2"
+        : "=&v"(a0), "=&v"(a1), "=&v"(a2), "=&v"(a3), "=&v"(a4), "=&v"(a5), "=&v"(a6), "=&v"(a7)
+        : "v"(r01), "v"(r2), "v"(w.w01[0]), "v"(w.w01[1]), "v"(w.w01[2]), "v"(w.w01[3]), "v"(w.w01[4]), "v"(w.w01[5]),
+          "v"(w.w01[6]), "v"(w.w01[7]), "v"(w.w2[0]), "v"(w.w2[1]), "v"(w.w2[2]), "v"(w.w2[3]), "v"(w.w2[4]),
+          "v"(w.w2[5]), "v"(w.w2[6]), "v"(w.w2[7]));
+    q[0] = pack_bf16x2(a0, a1); q[1] = pack_bf16x2(a2, a3); q[2] = pack_bf16x2(a4, a5); q[3] = pack_bf16x2(a6, a7);
 }
 
 __device__ __forceinline__ void unpack8(const uint4& w, float (&f)[8]) {
@@ -343,9 +405,10 @@ __global__ __launch_bounds__(kInterpWaves * 64) __attribute__((amdgpu_waves_per_
     const int K = p.K, dc = lane & 7, jg = lane >> 3;
 
     // to_q rows h*64 + 8 dc .. + 7 (three bf16 weights each: 48 bytes, 16-byte aligned)
-    float wq[24];
-    {
-        const bf16_t* wr = p.w_q + ((int64_t)h * 64 + 8 * dc) * 3;
+    const bf16_t* const wr = p.w_q + ((int64_t)h * 64 + 8 * dc) * 3;
+    float wq[RP ? 24 : 1];
+    QueryRows wp;
+    if constexpr (RP) {
         float t[8];
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
@@ -353,6 +416,8 @@ __global__ __launch_bounds__(kInterpWaves * 64) __attribute__((amdgpu_waves_per_
 #pragma unroll
             for (int e = 0; e < 8; ++e) wq[8 * c + e] = t[e];
         }
+    } else {
+        wp = query_rows(wr);
     }
     // per slot: the neighbour's row offsets and this lane's 8 query values,
     // q[j][d] = bf16(rel[j] . W[h*64 + d]) (fp32 sum of the three bf16 products: the
@@ -370,18 +435,29 @@ __global__ __launch_bounds__(kInterpWaves * 64) __attribute__((amdgpu_waves_per_
         const int64_t n = min(max(p.neighbors[sj], 0), p.S_from - 1);
         koff[i] = (Off)(2 * (n * p.k_sn + (int64_t)h * p.k_sh + 8 * dc));
         voff[i] = (Off)(2 * (n * p.v_sn + (int64_t)h * p.v_sh + 8 * dc));
-        const float r0 = round_bf16(p.rel_pos[3 * sj]), r1 = round_bf16(p.rel_pos[3 * sj + 1]),
-                    r2 = round_bf16(p.rel_pos[3 * sj + 2]);
+        if constexpr (RP) {
+            const float r0 = round_bf16(p.rel_pos[3 * sj]), r1 = round_bf16(p.rel_pos[3 * sj + 1]),
+                        r2 = round_bf16(p.rel_pos[3 * sj + 2]);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const uint32_t bits = __float_as_uint(round_bf16(fmaf(r2, wq[3 * e + 2], fmaf(r1, wq[3 * e + 1], r0 * wq[3 * e]))));
-            if constexpr (RP) qp[i][e] = (e & 1) ? bits : bits >> 16;
-            else if (e & 1) qp[i][e >> 1] |= bits;
-            else qp[i][e >> 1] = bits >> 16;
+            for (int e = 0; e < 8; ++e) {
+                const uint32_t bits = __float_as_uint(round_bf16(fmaf(r2, wq[3 * e + 2], fmaf(r1, wq[3 * e + 1], r0 * wq[3 * e]))));
+                qp[i][e] = (e & 1) ? bits : bits >> 16;
+            }
+        } else {
+            query_pairs(wp, pack_bf16x2(p.rel_pos[3 * sj], p.rel_pos[3 * sj + 1]), pack_bf16x2(p.rel_pos[3 * sj + 2], 0.f), qp[i]);
         }
     }
-    // the output dimension this lane ends up holding after the reduce-scatter
-    const int dout = 8 * dc + 4 * (lane >> 5) + 2 * ((lane >> 4) & 1) + ((lane >> 3) & 1);
+    // the output dimension this lane ends up holding: RP, after the reduce-scatter; else its own
+    const int dout = RP ? 8 * dc + 4 * (lane >> 5) + 2 * ((lane >> 4) & 1) + ((lane >> 3) & 1) : lane;
+    // fp32 products: this wave's rows of v (row j at byte 128 j) and its weights, in LDS
+    constexpr int kRows = 8 * NSLOT * 128, kWaveLds = kRows + 16 * NSLOT;
+    __shared__ __attribute__((aligned(16))) char v_lds[RP ? 16 : kInterpWaves * kWaveLds];
+    char* const vl = v_lds + (RP ? 0 : wave * kWaveLds);
+    uint32_t vaddr[2 * NSLOT];
+#pragma unroll
+    for (int g = 0; g < 2 * NSLOT; ++g)
+        vaddr[g] = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)vl +
+                   128 * knn_order<NSLOT>(4 * g + ((lane >> 2) & 3)) + 32 * (lane >> 4) + 8 * (lane & 3);
     bf16_t* out = p.out + ((int64_t)s * p.B * p.H + h) * 64 + dout;
 
     // k / v chunks of the current member; the next member's k is loaded as soon as the scores
@@ -402,7 +478,7 @@ __global__ __launch_bounds__(kInterpWaves * 64) __attribute__((amdgpu_waves_per_
         for (int i = 0; i < NSLOT; ++i) {
             float part;
             if constexpr (RP) part = chunk_sum(score_partial(qp[i], kw[i], ones));
-            else part = chunk_sum(score_dot(qp[i], kw[i]));
+            else part = dot_chunk_sum(score_dot(qp[i], kw[i]));
             // the score in base-2 units, sc = bf16(bf16(part) * scale) * log2 e.  A power-of-two
             // scale leaves bf16(part) * scale a bf16 value (a product too small to be normal is
             // below 2^-126 in magnitude, and so is the difference its rounding would make), so
@@ -430,14 +506,15 @@ __global__ __launch_bounds__(kInterpWaves * 64) __attribute__((amdgpu_waves_per_
         // each product is one dot product of (w, 0) or (0, w) with a packed pair of v.
         float acc[8];
         if constexpr (!RP) {
-            // fp32 products: one dot product each, accumulated slot by slot
+            // fp32 products: v and the weights through LDS, lane = dimension
+            float wt[NSLOT];
 #pragma unroll
             for (int i = 0; i < NSLOT; ++i) {
-                const float x = ex[i] * inv;
-                const uint32_t w_lo = pack_bf16x2(x, 0.f), w_hi = pack_bf16x2(0.f, x);
-                if (i == 0) out_fp32<true>(w_lo, w_hi, vw[i], acc);
-                else out_fp32<false>(w_lo, w_hi, vw[i], acc);
+                wt[i] = ex[i] * inv;
+                *reinterpret_cast<uint4*>(vl + 1024 * i + 16 * lane) = vw[i];
             }
+            put_weights(wt, vl + kRows, jg);
+            asm volatile("" ::: "memory");
         } else {
 #pragma unroll
         for (int i = 0; i < NSLOT; i += 2) {
@@ -466,6 +543,17 @@ __global__ __launch_bounds__(kInterpWaves * 64) __attribute__((amdgpu_waves_per_
 #pragma unroll
             for (int i = 0; i < NSLOT; ++i) vw[i] = ld_member<OFF32>(p.v + bn * p.v_sb, voff[i]);
         }
+        float o;
+        if constexpr (!RP) {
+            uint4 ww[NSLOT];
+            uint2 vv[2 * NSLOT];
+#pragma unroll
+            for (int i = 0; i < NSLOT; ++i) ww[i] = *reinterpret_cast<const uint4*>(vl + kRows + 16 * i);
+#pragma unroll
+            for (int g = 0; g < 2 * NSLOT; ++g) vv[g] = read_v4(vaddr[g]);
+            o = weighted_sum<NSLOT>(ww, vv);
+            asm volatile("" ::: "memory");
+        } else {
         // reduce-scatter over the 8 neighbour groups: halves (dims e / e + 4), row pairs
         // (e / e + 2), then lanes l ^ 8 (e / e + 1)
         float r4[4], r2[2];
@@ -475,29 +563,47 @@ __global__ __launch_bounds__(kInterpWaves * 64) __attribute__((amdgpu_waves_per_
         for (int e = 0; e < 2; ++e) r2[e] = swap16_add(r4[e], r4[e + 2]);
         const bool odd8 = lane & 8;
         const float keep = odd8 ? r2[1] : r2[0], give = odd8 ? r2[0] : r2[1];
-        const float o = keep + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(give), 0x128, 0xf, 0xf, false));
+        o = keep + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(give), 0x128, 0xf, 0xf, false));
+        }
         out[(int64_t)b * p.H * 64] = (bf16_t)(pack_bf16x2(o, 0.f) & 0xffffu);
     }
 }
 
-// LDS-staged form (fp32 products): one workgroup per (tile of up to 16 targets, head).  The
-// per-target kernel above issues 6 wave-wide 16-byte loads per (target, member, head), and at
-// one wave-instruction per ~32 cycles the texture addresser is then busy all the time; here
-// the tile's distinct source rows of k and v (the host-built tables) go into LDS once per
-// member with direct-to-LDS loads (lane l of an instruction lands at byte 16 l of a 1 KB run
-// of 8 rows), double-buffered, and the targets read them with ds_read_b128.  The arithmetic
-// per (target, member, head) is the fp32-product form of the kernel above in the same lane
-// layout and order, so both give the same bits.
+// LDS-staged form (fp32 products): one workgroup per (tile of up to 16 targets, group of hg
+// heads), passing over the group's heads and their members.  The tile's distinct source rows
+// of k and v (the host-built tables) go into LDS once per pass with direct-to-LDS loads (lane l
+// of an instruction lands at byte 16 l of a 1 KB run of 8 rows), double-buffered; waves 0 and 1
+// stage k, 2 and 3 v.  The arithmetic per (target, member, head) is the fp32-product form of
+// the kernel above in the same order, so both give the same bits.
+//
+// The bound is vector-instruction issue and LDS reads together (65 % and 61 % busy at 24
+// members), so the work per (target, member, head) is cut where it was the same in many lanes.
+// Each wave takes a quarter of the tile's targets (up to 4) together:
+//   scores   lane 8 jg + dc, as above, holds chunk dc of neighbours jg + 8 i of every target;
+//            the sums over the 8 chunk lanes leave target dc % 4's scores in lane (jg, dc), so
+//   softmax  one instruction sequence serves the wave's targets;
+//   output   lane = dimension: the weights go through LDS (the same in every lane), v comes
+//            through transposing LDS reads, four neighbours at once, and the matrix pipe sums
+//            over the neighbours (weighted_sum): no sum over lanes is left.
+// 24 members, lat-lon 121 x 240 -> HEALPix nside 64, 12 heads, K 24: 3324 -> 2503 us; one
+// member back: 268 -> 125 us.  Eight targets per wave and two waves (fewer instructions, but
+// two waves per SIMD): 2590 and 202 us.  Member groups as separate workgroups (for the L2's
+// sake) only repeat the prologue (4 us per workgroup): 2705 us at 8 members, 2990 at 4.
 //
 // LDS: per group of 8 rows, four 1 KB runs [k buffer 0][k buffer 1][v buffer 0][v buffer 1],
 // so a row's k and v in either buffer sit at fixed distances from its k in buffer 0 (the
-// reads take them as immediate offsets; the member loop is unrolled by two for the buffer).
-// Wave w takes targets t0 + w + 4 r of the tile and staging instructions w + 4 r over the k
-// groups, then the v groups.  One barrier per member: after it the next member's rows have
+// reads take them as immediate offsets; the pass is instantiated for either buffer); 16-byte
+// chunk c of v's row r sits at position c ^ (r & 6), which spreads the four rows of a
+// transposing read over the banks.  One barrier per pass: after it the next pass's rows have
 // landed (every wave waited for its own loads) and no wave still reads the buffer that the
-// next member's loads overwrite.
+// next pass's loads overwrite.
 __device__ __forceinline__ uint32_t lds_addr(const void* ptr) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)ptr;
+}
+__device__ __forceinline__ uint4 read_k(uint32_t lds) {
+    typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+    const v4u v = *(const __attribute__((address_space(3))) v4u*)(uintptr_t)lds;
+    return make_uint4(v[0], v[1], v[2], v[3]);
 }
 // address = base (uniform) + voff (per lane); LDS destination M0 + 16 l.  Inline assembly: the
 // compiler's own direct-to-LDS builtin makes it wait for these loads before every LDS read of
@@ -511,14 +617,10 @@ __device__ __forceinline__ void dma16(const void* base, uint32_t voff, uint32_t 
 #pragma clang diagnostic pop
 __device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// Three slots' scores (K 17..24, the model's 24) as one block: the three dot-product chains
-// interleaved, each from a literal 0 addend, accumulating through their own addend (no wait
-// between them); the three wait states a dot product's result needs before another VALU
-// instruction reads it; then the sums over the 8 chunk lanes of each neighbour group as DPP
-// adds (lanes l ^ 1, l ^ 2, then the half-row mirror), the three slots interleaved so each
-// DPP read of a register comes at least two instructions after its write.  Same products,
-// order and sums as chunk_sum(score_dot(...)) (the builtin form moves 0 into each
-// accumulator first, and two of its three half-mirror adds compiled to a move and an add).
+// Three slots' score partials (K 17..24, the model's 24) as one block: the three dot-product
+// chains interleaved, each from a literal 0 addend (the builtin form moves 0 into each
+// accumulator first), accumulating through their own addend (no wait between them); then the
+// three wait states a dot product's result needs before another VALU instruction reads it.
 __device__ __forceinline__ void score_dot3(const uint32_t (&q)[3][4], const uint4 (&k)[3], float (&a)[3]) {
     asm("v_dot2_f32_bf16 %0, %3, %15, 0\n\t"
         "v_dot2_f32_bf16 %1, %7, %19, 0\n\t"
@@ -532,68 +634,50 @@ __device__ __forceinline__ void score_dot3(const uint32_t (&q)[3][4], const uint
         "v_dot2_f32_bf16 %0, %6, %18, %0\n\t"
         "v_dot2_f32_bf16 %1, %10, %22, %1\n\t"
         "v_dot2_f32_bf16 %2, %14, %26, %2\n\t"
-        "s_nop 2\n\t"
-        "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-        "v_add_f32_dpp %1, %1, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-        "v_add_f32_dpp %2, %2, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-        "v_add_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-        "v_add_f32_dpp %1, %1, %1 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-        "v_add_f32_dpp %2, %2, %2 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-        "v_add_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-        "v_add_f32_dpp %1, %1, %1 row_half_mirror row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-        "v_add_f32_dpp %2, %2, %2 row_half_mirror row_mask:0xf bank_mask:0xf bound_ctrl:1"
+        "s_nop 2"
         : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2])
         : "v"(q[0][0]), "v"(q[0][1]), "v"(q[0][2]), "v"(q[0][3]), "v"(q[1][0]), "v"(q[1][1]), "v"(q[1][2]),
           "v"(q[1][3]), "v"(q[2][0]), "v"(q[2][1]), "v"(q[2][2]), "v"(q[2][3]), "v"(k[0].x), "v"(k[0].y),
           "v"(k[0].z), "v"(k[0].w), "v"(k[1].x), "v"(k[1].y), "v"(k[1].z), "v"(k[1].w), "v"(k[2].x), "v"(k[2].y),
           "v"(k[2].z), "v"(k[2].w));
 }
-// Three slots' weighted sum as one block: acc[2e] = sum_i (w_i, 0) . v_i[e], acc[2e + 1] =
-// sum_i (0, w_i) . v_i[e], slot by slot from a literal 0 addend (the order of
-// weighted_sum_fp32), then the three wait states.
-__device__ __forceinline__ void weighted_sum3(const uint32_t (&wl)[3], const uint32_t (&wh)[3], const uint4 (&v)[3],
-                                              float (&acc)[8]) {
-#define MOSAIC_PV_FIRST(W0, W1, X, Y, Z, T)        \
-    "v_dot2_f32_bf16 %0, " W0 ", " X ", 0\n\t"   \
-    "v_dot2_f32_bf16 %1, " W1 ", " X ", 0\n\t"   \
-    "v_dot2_f32_bf16 %2, " W0 ", " Y ", 0\n\t"   \
-    "v_dot2_f32_bf16 %3, " W1 ", " Y ", 0\n\t"   \
-    "v_dot2_f32_bf16 %4, " W0 ", " Z ", 0\n\t"   \
-    "v_dot2_f32_bf16 %5, " W1 ", " Z ", 0\n\t"   \
-    "v_dot2_f32_bf16 %6, " W0 ", " T ", 0\n\t"   \
-    "v_dot2_f32_bf16 %7, " W1 ", " T ", 0\n\t"
-#define MOSAIC_PV_NEXT(W0, W1, X, Y, Z, T)         \
-    "v_dot2_f32_bf16 %0, " W0 ", " X ", %0\n\t"  \
-    "v_dot2_f32_bf16 %1, " W1 ", " X ", %1\n\t"  \
-    "v_dot2_f32_bf16 %2, " W0 ", " Y ", %2\n\t"  \
-    "v_dot2_f32_bf16 %3, " W1 ", " Y ", %3\n\t"  \
-    "v_dot2_f32_bf16 %4, " W0 ", " Z ", %4\n\t"  \
-    "v_dot2_f32_bf16 %5, " W1 ", " Z ", %5\n\t"  \
-    "v_dot2_f32_bf16 %6, " W0 ", " T ", %6\n\t"  \
-    "v_dot2_f32_bf16 %7, " W1 ", " T ", %7\n\t"
-    asm(MOSAIC_PV_FIRST("%8", "%9", "%14", "%15", "%16", "%17")
-        MOSAIC_PV_NEXT("%10", "%11", "%18", "%19", "%20", "%21")
-        MOSAIC_PV_NEXT("%12", "%13", "%22", "%23", "%24", "%25")
-        "s_nop 2"
-        : "=&v"(acc[0]), "=&v"(acc[1]), "=&v"(acc[2]), "=&v"(acc[3]), "=&v"(acc[4]), "=&v"(acc[5]), "=&v"(acc[6]),
-          "=&v"(acc[7])
-        : "v"(wl[0]), "v"(wh[0]), "v"(wl[1]), "v"(wh[1]), "v"(wl[2]), "v"(wh[2]), "v"(v[0].x), "v"(v[0].y),
-          "v"(v[0].z), "v"(v[0].w), "v"(v[1].x), "v"(v[1].y), "v"(v[1].z), "v"(v[1].w), "v"(v[2].x), "v"(v[2].y),
-          "v"(v[2].z), "v"(v[2].w));
-#undef MOSAIC_PV_FIRST
-#undef MOSAIC_PV_NEXT
+
+constexpr int kTileWaves = 4;
+constexpr int kWaveTargets = kKnnTileTargets / kTileWaves;  // 4
+
+// The sums over the 8 chunk lanes of one slot's partials of 4 targets: lane dc of each
+// neighbour group gets target dc % 4's, in the tree of dot_chunk_sum: the half-row mirror, then
+// lanes l ^ 2 (even or odd pairs of targets kept) and l ^ 1 (one target kept).
+__device__ __forceinline__ float targets_chunk_sum(const float (&x)[kWaveTargets], int lane) {
+    float y[kWaveTargets];
+#pragma unroll
+    for (int e = 0; e < kWaveTargets; ++e) y[e] = dpp_add<0x141>(x[e]);
+    const bool b1 = lane & 2, b0 = lane & 1;
+    float z[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const float keep = b1 ? y[e + 2] : y[e], give = b1 ? y[e] : y[e + 2];
+        z[e] = keep + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(give), 0x4e, 0xf, 0xf, true));
+    }
+    const float keep = b0 ? z[1] : z[0], give = b0 ? z[0] : z[1];
+    return keep + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(give), 0xb1, 0xf, 0xf, true));
 }
 
-constexpr int kTileWaveTargets = kKnnTileTargets / kInterpWaves;     // 4
-constexpr int kTileWaveLoads = 2 * kKnnTileRows / 8 / kInterpWaves;  // 8 staging instructions per wave at most
+template <int N>
+using I = std::integral_constant<int, N>;
 
 template <int NSLOT, bool POW2>
-__global__ __launch_bounds__(kInterpWaves * 64) void knn_tile_kernel(InterpParams p, KnnTiles tl) {
+__global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu(NSLOT == 4 ? 2 : 3)))
+void knn_tile_kernel(InterpParams p, KnnTiles tl, int hg) {
+    constexpr int KP = 8 * NSLOT, WT = kWaveTargets, HW = kTileWaves / 2;
+    constexpr int kLoads = kKnnTileRows / 8 / HW;  // staging instructions per wave at most
     extern __shared__ __attribute__((aligned(16))) uint4 kv_lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int groups = (p.H + hg - 1) / hg;
     const int pair = xcd_remap(blockIdx.x, gridDim.x);
-    const int tile = pair / p.H, h = pair - tile * p.H;
+    const int tile = __builtin_amdgcn_readfirstlane(pair / groups);
+    const int h0 = __builtin_amdgcn_readfirstlane((pair - tile * groups) * hg), h1 = min(h0 + hg, p.H);
     const int K = p.K, dc = lane & 7, jg = lane >> 3;
     const int rows = tl.rows;
     // the tables are clamped into range (memory safety; a malformed table gives wrong rows)
@@ -601,124 +685,183 @@ __global__ __launch_bounds__(kInterpWaves * 64) void knn_tile_kernel(InterpParam
     const int t1 = __builtin_amdgcn_readfirstlane(min(max(tl.start[tile + 1], t0), min(t0 + kKnnTileTargets, p.S_to)));
     const int nsrc = __builtin_amdgcn_readfirstlane(min(max(tl.nsrc[tile], 1), rows));
     const int ng = (nsrc + 7) >> 3;  // 8-row groups per tensor
+    // this wave's targets
+    const int first = t0 + (t1 - t0) * wave / kTileWaves, nt = t0 + (t1 - t0) * (wave + 1) / kTileWaves - first;
 
-    // staging offsets: instruction r of this wave loads group gi = wave + 4 r (k groups, then v)
-    uint32_t soff[kTileWaveLoads];
-#pragma unroll
-    for (int r = 0; r < kTileWaveLoads; ++r) {
-        const int gi = wave + kInterpWaves * r;
-        const bool isv = gi >= ng;
-        const int row = 8 * (isv ? gi - ng : gi) + (lane >> 3);
-        const int n = min(max(tl.src[(int64_t)tile * rows + min(row, nsrc - 1)], 0), p.S_from - 1);
-        soff[r] = isv ? (uint32_t)(2 * (n * p.v_sn + (int64_t)h * p.v_sh + 8 * dc))
-                      : (uint32_t)(2 * (n * p.k_sn + (int64_t)h * p.k_sh + 8 * dc));
-    }
     const uint32_t lds0 = lds_addr(kv_lds);
-    auto stage = [&](int b, int buf) __attribute__((always_inline)) {
-        const char* kb = reinterpret_cast<const char*>(p.k + (int64_t)b * p.k_sb);
-        const char* vb = reinterpret_cast<const char*>(p.v + (int64_t)b * p.v_sb);
+    char* const mem = reinterpret_cast<char*>(kv_lds);
+    // after the staging buffers, per wave: rel (bf16: 8 bytes per target and neighbour), the
+    // weight tables and the neighbours' rows (LDS offsets)
+    char* const rel_lds = mem + 512 * rows + wave * (WT * KP * 12);
+    char* const w_lds = rel_lds + WT * KP * 8;
+    char* const row_lds = w_lds + WT * KP * 2;
+
+    // the first half of the waves stage k, the second v: instruction r of a wave stages 8-row
+    // group g0 + HW r of its tensor
+    const bool isv = wave >= HW;
+    const int g0 = wave & (HW - 1);
+    const bf16_t* const src = isv ? p.v : p.k;
+    const int64_t s_n = isv ? p.v_sn : p.k_sn, s_b = isv ? p.v_sb : p.k_sb, s_h = isv ? p.v_sh : p.k_sh;
+    uint32_t soff[kLoads];
 #pragma unroll
-        for (int r = 0; r < kTileWaveLoads; ++r) {
-            const int gi = wave + kInterpWaves * r;
-            if (gi >= 2 * ng) break;  // uniform
-            const bool isv = gi >= ng;
-            const uint32_t dst = lds0 + (uint32_t)(4 * (isv ? gi - ng : gi) + 2 * isv + buf) * 1024u;
-            if (isv) dma16(vb, soff[r], __builtin_amdgcn_readfirstlane(dst));
-            else dma16(kb, soff[r], __builtin_amdgcn_readfirstlane(dst));
+    for (int r = 0; r < kLoads; ++r) {
+        // the whole table row, so that these loads do not wait for nsrc
+        const int row = min(8 * (g0 + HW * r) + jg, rows - 1);
+        const int n = min(max(tl.src[(int64_t)tile * rows + row], 0), p.S_from - 1);
+        soff[r] = (uint32_t)(2 * (n * s_n + 8 * (isv ? dc ^ (jg & 6) : dc)));
+    }
+    auto stage = [&](int h, int b, int buf) __attribute__((always_inline)) {
+        const bf16_t* base = src + (int64_t)b * s_b + (int64_t)h * s_h;
+        const uint32_t dst = lds0 + 4096u * g0 + (uint32_t)(2 * isv + buf) * 1024u;
+#pragma unroll
+        for (int r = 0; r < kLoads; ++r) {
+            if (g0 + HW * r >= ng) break;  // uniform
+            dma16(base, soff[r], __builtin_amdgcn_readfirstlane(dst + 4096u * HW * r));
         }
     };
+    stage(h0, 0, 0);
 
-    // to_q rows h*64 + 8 dc .. + 7
-    float wq[24];
-    {
-        const bf16_t* wr = p.w_q + ((int64_t)h * 64 + 8 * dc) * 3;
-        float t[8];
+    // this wave's targets: rel and row offsets into LDS, target indices
+    for (int x = lane; x < WT * KP; x += 64) {
+        const int pos = min(first + x / KP, p.S_to - 1), j = min(x % KP, K - 1);
+        const int s = p.target_order ? min(max(p.target_order[pos], 0), p.S_to - 1) : pos;
+        const int sl = min(max(tl.slot[(int64_t)pos * K + j], 0), rows - 1);
+        const float* r = p.rel_pos + 3 * ((int64_t)s * K + j);
+        reinterpret_cast<uint2*>(rel_lds)[x] = make_uint2(pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], 0.f));
+        reinterpret_cast<uint16_t*>(row_lds)[x] = (uint16_t)(4096 * (sl >> 3) + 128 * (sl & 7));
+    }
+    int tgt[WT];
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            unpack8(ld16(wr + 8 * c), t);
+    for (int r = 0; r < WT; ++r) {
+        const int pos = min(first + r, p.S_to - 1);
+        tgt[r] = __builtin_amdgcn_readfirstlane(p.target_order ? min(max(p.target_order[pos], 0), p.S_to - 1) : pos);
+    }
+    wait_vmem();
+    __syncthreads();
+    // LDS addresses in buffer 0: k chunk dc of neighbours jg + 8 i; v, as read_v4 takes them
+    uint32_t kaddr[WT][NSLOT], vaddr[WT][2 * NSLOT];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) wq[8 * c + e] = t[e];
+    for (int r = 0; r < WT; ++r) {
+        const uint16_t* row = reinterpret_cast<const uint16_t*>(row_lds) + r * KP;
+#pragma unroll
+        for (int i = 0; i < NSLOT; ++i) kaddr[r][i] = lds0 + row[jg + 8 * i] + 16 * dc;
+#pragma unroll
+        for (int g = 0; g < 2 * NSLOT; ++g) {
+            const uint32_t o = row[knn_order<NSLOT>(4 * g + ((lane >> 2) & 3))];
+            vaddr[r][g] = lds0 + o + ((((uint32_t)lane >> 4) ^ ((o >> 8) & 3)) << 5) + 8 * (lane & 3);
         }
     }
-    // per target of this wave: its index, its slots' k rows in buffer 0 (LDS byte offsets) and
-    // its query pairs
-    int tgt[kTileWaveTargets];
-    uint32_t koff[kTileWaveTargets][NSLOT];
-    uint32_t qp[kTileWaveTargets][NSLOT][4];
+
+    // opaque from here: kept as sums of two registers each otherwise
 #pragma unroll
-    for (int r = 0; r < kTileWaveTargets; ++r) {
-        const int pos = min(t0 + wave + kInterpWaves * r, p.S_to - 1);
-        const int s = __builtin_amdgcn_readfirstlane(p.target_order ? min(max(p.target_order[pos], 0), p.S_to - 1) : pos);
-        tgt[r] = s;
+    for (int r = 0; r < WT; ++r) {
+#pragma unroll
+        for (uint32_t& a : kaddr[r]) asm volatile("" : "+v"(a));
+#pragma unroll
+        for (uint32_t& a : vaddr[r]) asm volatile("" : "+v"(a));
+    }
+
+    uint32_t qp[WT][NSLOT][4];
+    // pass (h, b) from buffer BUF (the next pass staged into the other one meanwhile)
+    auto pass = [&](int h, int b, auto BUF) __attribute__((always_inline)) {
+        constexpr int buf = decltype(BUF)::value;
+        const bool last = b + 1 == p.B;
+        if (!last || h + 1 < h1) stage(last ? h + 1 : h, last ? 0 : b + 1, buf ^ 1);
+        // targets [R0, R1) at a time, the next target's rows read before this one's products
+        float part[NSLOT][WT];
+        auto scores = [&](auto R0, auto R1) __attribute__((always_inline)) {
+            constexpr int r0 = decltype(R0)::value, r1 = decltype(R1)::value;
+            uint4 kw[2][NSLOT];
+            auto fetch = [&](int r) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < NSLOT; ++i) kw[r & 1][i] = read_k(kaddr[r][i] + 1024 * buf);
+            };
+            fetch(r0);
+#pragma unroll
+            for (int r = r0; r < r1; ++r) {
+                if (r + 1 < r1) fetch(r + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (NSLOT == 3) {
+                    float a[3];
+                    score_dot3(qp[r], kw[r & 1], a);
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) part[i][r] = a[i];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < NSLOT; ++i) part[i][r] = score_dot(qp[r][i], kw[r & 1][i]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < NSLOT; ++i)
+#pragma unroll
+            for (int r = 2; r < WT; ++r) part[i][r] = 0.f;
+        scores(I<0>{}, I<2>{});
+        if (nt > 2) scores(I<2>{}, I<3>{});
+        if (nt > 3) scores(I<3>{}, I<4>{});
+        // the first target's values are on their way during the softmax
+        uint2 vv[2][2 * NSLOT];
+        auto fetch_v = [&](int r) __attribute__((always_inline)) {
+#pragma unroll
+            for (int g = 0; g < 2 * NSLOT; ++g) vv[r & 1][g] = read_v4(vaddr[r][g], 2048 + 1024 * buf);
+        };
+        fetch_v(0);
+        __builtin_amdgcn_sched_barrier(0);
+        float sc[NSLOT], wt[NSLOT], m;
 #pragma unroll
         for (int i = 0; i < NSLOT; ++i) {
-            const int j = min(jg + 8 * i, K - 1);
-            const int sl = min(max(tl.slot[(int64_t)pos * K + j], 0), rows - 1);
-            koff[r][i] = lds0 + (uint32_t)(4096 * (sl >> 3) + 128 * (sl & 7) + 16 * dc);
-            const int64_t sj = (int64_t)s * K + j;
-            const float r0 = round_bf16(p.rel_pos[3 * sj]), r1 = round_bf16(p.rel_pos[3 * sj + 1]),
-                        r2 = round_bf16(p.rel_pos[3 * sj + 2]);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const uint32_t bits = __float_as_uint(round_bf16(fmaf(r2, wq[3 * e + 2], fmaf(r1, wq[3 * e + 1], r0 * wq[3 * e]))));
-                if (e & 1) qp[r][i][e >> 1] |= bits;
-                else qp[r][i][e >> 1] = bits >> 16;
-            }
+            const float t = scaled_score<POW2>(targets_chunk_sum(part[i], lane), p);
+            sc[i] = i < NSLOT - 1 || jg + 8 * i < K ? t : -INFINITY;
+            m = i == 0 ? sc[0] : fmaxf(m, sc[i]);
         }
-    }
-    const int dout = 8 * dc + 4 * (lane >> 5) + 2 * ((lane >> 4) & 1) + ((lane >> 3) & 1);
-
-    // member b from buffer BUF (member b + 1 staged into the other one meanwhile)
-    auto member = [&](int b, auto BUF) __attribute__((always_inline)) {
-        constexpr int buf = decltype(BUF)::value;
-        if (b + 1 < p.B) stage(b + 1, buf ^ 1);
-        const char* lds = reinterpret_cast<const char*>(kv_lds) - lds0;  // koff holds absolute LDS addresses
+        softmax_weights(sc, m, wt);
+        put_weights(wt, w_lds + (dc & (WT - 1)) * (KP * 2), jg);
+        asm volatile("" ::: "memory");
+        // outputs likewise
+        auto outputs = [&](auto R0, auto R1) __attribute__((always_inline)) {
+            constexpr int r0 = decltype(R0)::value, r1 = decltype(R1)::value;
+            uint4 ww[2][NSLOT];
+            auto fetch = [&](int r) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < kTileWaveTargets; ++r) {
-            if (t0 + wave + kInterpWaves * r >= t1) break;  // uniform
-            uint4 kw[NSLOT], vw[NSLOT];
+                for (int i = 0; i < NSLOT; ++i) ww[r & 1][i] = *reinterpret_cast<const uint4*>(w_lds + r * (KP * 2) + 16 * i);
+                if (r > 0) fetch_v(r);
+            };
+            fetch(r0);
 #pragma unroll
-            for (int i = 0; i < NSLOT; ++i) {
-                kw[i] = *reinterpret_cast<const uint4*>(lds + koff[r][i] + 1024 * buf);
-                vw[i] = *reinterpret_cast<const uint4*>(lds + koff[r][i] + 2048 + 1024 * buf);
+            for (int r = r0; r < r1; ++r) {
+                if (r + 1 < r1) fetch(r + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                const float o = weighted_sum<NSLOT>(ww[r & 1], vv[r & 1]);
+                bf16_t* orow = p.out + (((int64_t)tgt[r] * p.B + b) * p.H + h) * 64;  // uniform
+                // targets past the wave's last: a store of no lane's
+                const auto rs = __builtin_amdgcn_make_buffer_rsrc(orow, (short)0, r < nt ? 128 : 0, 0x00020000);
+                __builtin_amdgcn_raw_buffer_store_b16((bf16_t)(pack_bf16x2(o, 0.f) & 0xffffu), rs, 2 * lane, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            float part[NSLOT], sc[NSLOT], m;
-            if constexpr (NSLOT == 3) {
-                score_dot3(qp[r], kw, part);
-            } else {
-#pragma unroll
-                for (int i = 0; i < NSLOT; ++i) part[i] = score_dot(qp[r][i], kw[i]);
-            }
-#pragma unroll
-            for (int i = 0; i < NSLOT; ++i) {
-                const float sum = NSLOT == 3 ? part[i] : chunk_sum(part[i]);  // score_dot3 sums the chunk lanes itself
-                sc[i] = i < NSLOT - 1 || jg + 8 * i < K ? scaled_score<POW2>(sum, p) : -INFINITY;
-                m = i == 0 ? sc[0] : fmaxf(m, sc[i]);
-            }
-            float wt[NSLOT], acc[8];
-            softmax_weights(sc, m, wt);
-            if constexpr (NSLOT == 3) {
-                uint32_t wl[3], wh[3];
-#pragma unroll
-                for (int i = 0; i < 3; ++i) { wl[i] = pack_bf16x2(wt[i], 0.f); wh[i] = pack_bf16x2(0.f, wt[i]); }
-                weighted_sum3(wl, wh, vw, acc);
-            } else {
-                weighted_sum_fp32(wt, vw, acc);
-            }
-            const float o = reduce_scatter(acc, lane);
-            bf16_t* orow = p.out + (((int64_t)tgt[r] * p.B + b) * p.H + h) * 64;  // uniform
-            orow[dout] = (bf16_t)(pack_bf16x2(o, 0.f) & 0xffffu);
-        }
-        wait_vmem();
+        };
+        outputs(I<0>{}, I<2>{});
+        if (nt > 2) outputs(I<2>{}, I<3>{});
+        if (nt > 3) outputs(I<3>{}, I<4>{});
+        // the staging loads are older than the outputs' stores, of which there are two at least
+        asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
         __syncthreads();
     };
 
-    stage(0, 0);
-    wait_vmem();
-    __syncthreads();
-    for (int b = 0; b < p.B; b += 2) {
-        member(b, std::integral_constant<int, 0>{});
-        if (b + 1 < p.B) member(b + 1, std::integral_constant<int, 1>{});
+    int buf = 0;
+    for (int h = h0; h < h1; ++h) {
+        const QueryRows wr = query_rows(p.w_q + ((int64_t)h * 64 + 8 * dc) * 3);
+#pragma unroll
+        for (int r = 0; r < WT; ++r)
+#pragma unroll
+            for (int i = 0; i < NSLOT; ++i) {
+                const uint2 rel = reinterpret_cast<const uint2*>(rel_lds)[r * KP + jg + 8 * i];
+                query_pairs(wr, rel.x, rel.y, qp[r][i]);
+            }
+        for (int b = 0; b < p.B; ++b, buf ^= 1) {
+            if (buf) pass(h, b, std::integral_constant<int, 1>{});
+            else pass(h, b, std::integral_constant<int, 0>{});
+        }
     }
 }
 
@@ -766,10 +909,20 @@ bool knn_tiled_supported(const InterpParams& p) { return !p.round_products && kn
 
 hipError_t launch_knn_attn_tiled(const InterpParams& p, const KnnTiles& t, hipStream_t s) {
     if (!knn_tiled_supported(p) || t.rows <= 0 || t.rows % 8 || t.rows > kKnnTileRows) return hipErrorInvalidValue;
-    const int64_t wgs = (int64_t)t.n * p.H;
+    // heads per workgroup: 48 passes (heads times members) make a workgroup's prologue (the
+    // tables, 4 us of chained loads) small, but 2048 workgroups are left to fill the chip's 768
+    // slots evenly (the model's grids, 12 heads: one member 218 us at 1 head, 120 at 12; 24
+    // members 2604 at 1, 2469 at 2, 2678 at 12; 563 tiles, 4 heads, 24 members: 179 at 1 head,
+    // 191 at 2); a grid smaller than that takes one round of the slots (68 tiles, 12 heads, one
+    // member: 28 us at 1 head, 21 at 2)
+    const int64_t work = (int64_t)t.n * p.H;
+    const int64_t fill = work < 2048 ? (work + 767) / 768 : work / 2048;
+    int hg = (int)max((int64_t)1, min(min((int64_t)(48 + p.B - 1) / p.B, fill), (int64_t)p.H));
+    hg = (p.H + (p.H + hg - 1) / hg - 1) / ((p.H + hg - 1) / hg);  // groups as equal as they get
+    const int64_t wgs = (int64_t)t.n * ((p.H + hg - 1) / hg);
     if (wgs <= 0) return hipSuccess;
     if (wgs > 0x7fffffff) return hipErrorInvalidValue;
-    void* args[] = {const_cast<InterpParams*>(&p), const_cast<KnnTiles*>(&t)};
+    void* args[] = {const_cast<InterpParams*>(&p), const_cast<KnnTiles*>(&t), &hg};
     const void* fn = nullptr;
     switch ((p.K + 7) / 8) {
         case 1: fn = p.scale_pow2 ? (const void*)&knn_tile_kernel<1, true> : (const void*)&knn_tile_kernel<1, false>; break;
@@ -778,8 +931,10 @@ hipError_t launch_knn_attn_tiled(const InterpParams& p, const KnnTiles& t, hipSt
         case 4: fn = p.scale_pow2 ? (const void*)&knn_tile_kernel<4, true> : (const void*)&knn_tile_kernel<4, false>; break;
         default: return hipErrorInvalidValue;
     }
-    const size_t lds = 4u * (size_t)t.rows * 128u;  // per 8-row group: k and v, two buffers each
-    return hipLaunchKernel(fn, dim3((unsigned)wgs), dim3(kInterpWaves * 64), args, lds, s);
+    // per row: k and v, two buffers each; then the waves' tables (12 bytes per target and
+    // neighbour)
+    const size_t lds = 512u * (size_t)t.rows + (size_t)kKnnTileTargets * 8u * ((p.K + 7) / 8) * 12u;
+    return hipLaunchKernel(fn, dim3((unsigned)wgs), dim3(kTileWaves * 64), args, lds, s);
 }
 
 }  // namespace mosaic

@@ -442,3 +442,33 @@ def test_knn_attention_tiled_head_and_member_counts(H, B):
     tiled = knn_attention(*args, target_order=order.to(DEV), tiles=tiles_on(nb, order))
     assert torch.equal(tiled, direct)
     close(tiled, oracle(k, v, nb, rel, w_q, 0.125, False))
+
+
+@pytest.mark.parametrize("K,H,B", [(24, 21, 1), (24, 21, 3), (8, 40, 2), (17, 21, 2), (32, 21, 1)])
+def test_knn_attention_tiled_head_groups(K, H, B):
+    """Workgroups that pass over several heads: groups of unequal size, odd pass counts (the
+    staging buffers alternate across heads), one to four neighbour slots.  Bit for bit the
+    per-target kernel; an infinite value reaches the targets that list its source, and no other
+    target or dimension."""
+    ll, hp = lonlat_grid(24, 13), torch.deg2rad(get_healpix_grid(8))
+    nb, rel = scheme(ll, hp, K)
+    k, v = rand(len(ll), B, H, 64, seed=150 + K), rand(len(ll), B, H, 64, seed=160 + B)
+    w_q = rand(H * 64, 3, seed=170)
+    order = spatial_order(hp)
+    tiles = tiles_on(nb, order)
+    assert 768 < (tiles["start"].numel() - 1) * H    # more (tile, head) pairs than one round of workgroups
+
+    def both(v):
+        args = (k.to(DEV), v.to(DEV), nb.to(DEV), rel.to(DEV), w_q.to(DEV), 0.125)
+        return (knn_attention(*args, target_order=order.to(DEV)).cpu(),
+                knn_attention(*args, target_order=order.to(DEV), tiles=tiles).cpu())
+    direct, tiled = both(v)
+    assert torch.equal(tiled, direct)
+    close(tiled, oracle(k, v, nb, rel, w_q, 0.125, False))
+    v[100, 0, H - 1, 37] = float("inf")
+    inf_direct, inf_tiled = both(v)
+    hit = torch.zeros(len(hp), B, H, 64, dtype=torch.bool)
+    hit[(nb == 100).any(1), 0, H - 1, 37] = True
+    for out in (inf_direct, inf_tiled):
+        assert torch.equal(out[~hit], direct[~hit])
+        assert not torch.isfinite(out[hit]).any()
