@@ -365,11 +365,15 @@ void bwd_dq_kernel(BwdParams p, int head_groups, int total_wgs) {
 // memory straight into LDS: a ring of three slots, loads requested two steps ahead, one barrier
 // per step.  All tiles use the bwd_swz layout.  The two waves of a key half sum their partial
 // dV^T / dK^T once, at the end.
-__global__ __attribute__((amdgpu_flat_work_group_size(256, 256)))
+//
+// Three workgroups per CU (168 registers; 51.7 KB of LDS, the K and V tiles having no buffer of
+// their own): a step is a chain of LDS reads, products, exponentials and products, and two
+// waves per SIMD left it half uncovered.  The grid is often a small multiple of the 256 CUs,
+// where the third slot also fills the last round.  Nside 32, 128-token blocks, 16/4 heads (3
+// workgroups per CU): 230 -> 191 us against two per CU; Nside 64, 64-token blocks, 12/3 heads: the
+// forward and backward 823 -> 798 us.
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(3, 3)))
 void bwd_dkv_kernel(BwdParams p) {
-    __shared__ __attribute__((aligned(1024))) bf16_t kvs[2 * kTileElems];   // K tile, V tile
-    bf16_t* Ks = kvs;
-    bf16_t* Vs = kvs + kTileElems;
     // Three steps in a ring; a slot holds the step's q' tile, do tile, then -lse and -delta of
     // its 64 rows (fp32).  The loop below is unrolled over the slots (each an array of its own)
     // and its loads are issued as inline assembly, so no compiler-inserted wait holds a step's
@@ -378,6 +382,10 @@ void bwd_dkv_kernel(BwdParams p) {
     constexpr int kSlotElems = 2 * kTileElems + 256;
     __shared__ __attribute__((aligned(1024))) bf16_t ring0[kSlotElems], ring1[kSlotElems], ring2[kSlotElems];
     __shared__ uint64_t mark[kMaxBwdBlocks / 64];   // bit t: query block t selected this block
+    // The K and V tiles pass through slot 2 on their way to registers: its first step is requested
+    // behind the first round's barrier, which retires every wave's reads of them.
+    bf16_t* Ks = ring2;
+    bf16_t* Vs = ring2 + kTileElems;
     // key tiles in XCD-contiguous ranges: with selections that follow spatial proximity,
     // neighbouring key tiles are selected by the same query blocks and share their (q', do)
     // tiles in one L2

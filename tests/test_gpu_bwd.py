@@ -60,6 +60,21 @@ def test_sparse_attn_bwd_matches_oracle(B, N, Hq, Hk, bs, K):
         check(gg, rr, name)
 
 
+@pytest.mark.parametrize("G", [1, 2, 3, 4])
+def test_sparse_attn_bwd_few_steps(G):
+    """Key tiles with the fewest steps of the grad-k/v ring (its K and V pass through a slot of it):
+    0, 1, 2 and 5 selecting query blocks of G heads each."""
+    print(f"bwd few steps G={G}", flush=True)
+    q, k, v, do, _ = case(G, 1, 512, G, 1, 64, 1)
+    idx = torch.tensor([1, 2, 2, 5, 5, 5, 5, 5]).view(1, 8, 1, 1)
+    qd, kd, vd, dod, idxd = (t.to(DEV) for t in (q, k, v, do, idx))
+    o, lse = mosaic_attn_fwd(qd, kd, vd, idxd, 64, 0.125)
+    grads = mosaic_attn_bwd(qd, kd, vd, o, lse, dod, 0.125, idxd, 64)
+    refs = O.sparse_attn_bwd(q, k, v, o.cpu(), lse.cpu(), do, idx, 64, 0.125)
+    for name, gg, rr in zip(("dq", "dk", "dv"), grads, refs):
+        check(gg, rr, name)
+
+
 @pytest.mark.parametrize("B,nside,Hq,Hk,K,nsample", [(1, 64, 12, 3, 16, 8), (4, 32, 16, 4, 16, 4)],
                          ids=["nside64", "nside32_b4"])
 def test_sparse_attn_bwd_full_size_sampled(B, nside, Hq, Hk, K, nsample):
