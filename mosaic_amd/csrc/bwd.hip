@@ -5,13 +5,18 @@
 // arithmetic and rounding points:
 //   q'    = bf16((q * scale) * log2 e)                      (ops.py:236-237, 412-414)
 //   delta = bf16(sum_d bf16(o * do))                        (ops.py:458, eager bf16 ops)
-//   dq    = bf16(((sum over selected keys of bf16(P ln2 (dP - delta)) k) * scale) * log2 e)
+//   dq    = bf16((sum over selected keys of bf16(P (dP - delta)) k) * scale)
 //           with P = exp2(q'.k - lse), dP = do.v            (ops.py:265-273)
 //   dv    = sum over the queries that selected the key of bf16(P) do
-//   dk    = sum of bf16(P (dP - delta) ln2) q'              (ops.py:425-431)
-// Products run on v_mfma_f32_32x32x16_bf16 with fp32 accumulation.  One difference in order:
+//   dk    = (sum of bf16(P (dP - delta)) q') * ln2          (ops.py:425-431)
+// Products run on v_mfma_f32_32x32x16_bf16 with fp32 accumulation.  Two differences in order:
 // grad k/v accumulates S and dP onto -lse and -delta, so those subtractions happen inside the
-// fp32 accumulation rather than after it.
+// fp32 accumulation rather than after it; and the factor ln2 of dS multiplies the fp32 sums (in dq
+// it cancels the factor log2 e) rather than every element before its rounding to bf16.  That is one
+// multiplication less per element of kernels whose vector pipe is as loaded as the matrix
+// cores, and no rounding more: error against 64 bits 0.0034 before and after, grad q 152 -> 140 us
+// at Nside 32 with 128-token blocks and 16/4 heads, 304 -> 293 us at Nside 64, 64-token blocks, 12/3 heads
+// (grad k/v 191 -> 188 and unchanged).
 //
 // The reference's grad-k/v program scans a dense [B, Hk, nb, nb] boolean block mask for every
 // key block.  Here each key-tile workgroup marks, in LDS, the query blocks whose selection row
@@ -64,7 +69,7 @@ typedef short v4i16 __attribute__((ext_vector_type(4)));
 // registers):
 //   S^T  = K Q'^T          A = K rows (b128 reads),  B = q' fragments (registers)
 //   dP^T = V dO^T          A = V rows,               B = do fragments (registers)
-//   dS   = bf16(exp2(S - lse) ln2 (dP - delta)), packed in accumulator order as B operands
+//   dS   = bf16(exp2(S - lse) (dP - delta)), packed in accumulator order as B operands
 //   dQ^T += K^T dS^T       A = K^T (transposing ds_read_b64_tr_b16 reads of the K tile)
 // Both tiles use the bwd_swz layout.
 constexpr int kTileElems = 64 * 64;
@@ -299,8 +304,8 @@ void bwd_dq_kernel(BwdParams p, int head_groups, int total_wgs) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const int e0 = 8 * s2 + 2 * i;
-                        const float p0 = __builtin_amdgcn_exp2f(s[qt][e0] - lse[qt]) * kLn2;
-                        const float p1 = __builtin_amdgcn_exp2f(s[qt][e0 + 1] - lse[qt]) * kLn2;
+                        const float p0 = __builtin_amdgcn_exp2f(s[qt][e0] - lse[qt]);
+                        const float p1 = __builtin_amdgcn_exp2f(s[qt][e0 + 1] - lse[qt]);
                         w4[i] = pack_bf16x2(p0 * (dp[qt][e0] - dlt[qt]), p1 * (dp[qt][e0 + 1] - dlt[qt]));
                     }
                     db[qt][s2] = as_bf16x8(make_uint4(w4[0], w4[1], w4[2], w4[3]));
@@ -335,7 +340,7 @@ void bwd_dq_kernel(BwdParams p, int head_groups, int total_wgs) {
         if (t + 2 < total) tile_dma<NW>(dk, dv, kb, vb, p.k_sn, p.v_sn, next_key0(), Ks0, Vs0, wave);
         if (t + 1 < total) tile(Ks1, Vs1);
     }
-    // dq = bf16((dQ scale) log2 e), rows n0 + 32 qt + r, dims 32 dt + 8 g4 + 4 hh + 0..3
+    // dq = bf16(dQ scale), rows n0 + 32 qt + r, dims 32 dt + 8 g4 + 4 hh + 0..3
     bf16_t* out = p.dq + (((int64_t)b * p.N + n0) * p.Hq + j) * 64;
 #pragma unroll
     for (int qt = 0; qt < 2; ++qt)
@@ -345,8 +350,8 @@ void bwd_dq_kernel(BwdParams p, int head_groups, int total_wgs) {
             for (int g4 = 0; g4 < 4; ++g4) {
                 const f32x16& a = acc[dt][qt];
                 uint2 w2;
-                w2.x = pack_bf16x2((a[4 * g4 + 0] * p.scale) * kLog2e, (a[4 * g4 + 1] * p.scale) * kLog2e);
-                w2.y = pack_bf16x2((a[4 * g4 + 2] * p.scale) * kLog2e, (a[4 * g4 + 3] * p.scale) * kLog2e);
+                w2.x = pack_bf16x2(a[4 * g4 + 0] * p.scale, a[4 * g4 + 1] * p.scale);
+                w2.y = pack_bf16x2(a[4 * g4 + 2] * p.scale, a[4 * g4 + 3] * p.scale);
                 *reinterpret_cast<uint2*>(out + (int64_t)(32 * qt + r) * p.Hq * 64 + 32 * dt + 8 * g4 + 4 * hh) = w2;
             }
 }
@@ -359,7 +364,7 @@ void bwd_dq_kernel(BwdParams p, int head_groups, int total_wgs) {
 // dV^T += do^T P and dK^T += q'^T dS with k running over those query rows; the A operands
 // (do^T, q'^T) come from transposing LDS reads of the row-major tiles in the same row order.
 // The wave's K and V rows stay in registers for all steps.  S and dP accumulate onto -lse and
-// -delta of their rows (written by the grad-q kernel), so P = exp2(S) and dS = P dP ln2 take
+// -delta of their rows (written by the grad-q kernel), so P = exp2(S) and dS = P dP take
 // no subtraction (the subtraction happens inside the fp32 accumulation instead of after it).
 // The step's q' rows (pre-scaled by the grad-q kernel), do rows, -lse and -delta go from global
 // memory straight into LDS: a ring of three slots, loads requested two steps ahead, one barrier
@@ -533,7 +538,7 @@ void bwd_dkv_kernel(BwdParams p) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) {   // s = q'.k - lse, dp = do.v - delta
             const float pr = __builtin_amdgcn_exp2f(s[e]);
-            const float ds = pr * dp[e] * kLn2;
+            const float ds = pr * dp[e];
             pb[e >> 3][e & 7] = (__bf16)pr;
             db[e >> 3][e & 7] = (__bf16)ds;
         }
@@ -610,7 +615,7 @@ void bwd_dkv_kernel(BwdParams p) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int e = 4 * g + i;
-                    kx[i] = dkT[dblk][e] + red[32 * (16 * dblk + e)];
+                    kx[i] = (dkT[dblk][e] + red[32 * (16 * dblk + e)]) * kLn2;
                     vx[i] = dvT[dblk][e] + red[32 * (32 + 16 * dblk + e)];
                 }
                 const int d = 32 * dblk + 8 * g + 4 * hh;
