@@ -217,7 +217,8 @@ __global__ __launch_bounds__(kPoolMaxThreads<ROPE>) void pool_kernel(PoolParams 
 // go to workgroups of their own.  Pass alone, 1 thread -> the split: Nside 16, 20/5 heads 6.7 ->
 // 4.9 us (180 -> 1440 waves), Nside 32, 12/3 heads 7.5 -> 5.8 us, 16/4 heads with 128-token
 // blocks 13.4 -> 8.4 us, that shape's keys alone 11.7 -> 4.1 us; with RoPE the whole op there
-// 118 -> 109 us.  At Nside 64 splitting only adds the sums' exchange (18.6 -> 19.3 us at four
+// 118 -> 109 us.  With RoPE and 768 waves or more, only to runs of 32 tokens: 24,576 tokens in
+// 64-token blocks, 12/3 heads (864 waves), whole op 86.9 us at two threads, 87.4 at four.  At Nside 64 splitting only adds the sums' exchange (18.6 -> 19.3 us at four
 // threads).  The largest passes (24 members) stream from HBM and gain from two threads and
 // smaller workgroups again: 176 -> 167 us (8 members: 48.4 -> 51.3 us, so not there).
 struct PoolShape { int tpc, wg; };
@@ -227,7 +228,8 @@ PoolShape pool_shape(const PoolParams& p, int chunks) {
     const bool rope = p.rope_cos != nullptr;
     int tpc = rope ? 2 : 1;
     const int first = tpc;
-    while (tpc < 8 && waves * tpc < (rope ? 3072 : 768) && p.bs >= 16 * tpc) tpc *= 2;
+    const int run = rope && waves >= 768 ? 64 : 16;
+    while (tpc < 8 && waves * tpc < (rope ? 3072 : 768) && p.bs >= run * tpc) tpc *= 2;
     return {tpc, tpc > first ? (rope ? 256 : 128) : 0};
 }
 
