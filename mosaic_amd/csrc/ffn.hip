@@ -22,11 +22,12 @@
 //    SIMD one wave issues LDS reads and loads while the other one feeds the matrix cores;
 //  - persistent workgroups: the loads of a tile's first iterations are issued during the tile
 //    before it, so no tile starts on an empty pipeline, and the epilogue runs over them;
-//  - hardware exp2 and reciprocal in the gate (1 ulp in fp32, before its rounding to bf16).
-// Measured (24 members, 1,179,648 rows): 768 -> 2 x 3072 in 9.28 ms, against 13.76 ms for the
+//  - hardware exp2 and reciprocal in the gate, arranged so that silu rounds to the same bf16 value
+//    as with expf and a division for every bf16 argument (gate).
+// Measured (24 members, 1,179,648 rows): 768 -> 2 x 3072 in 9.40 ms, against 13.76 ms for the
 // library GEMM and the gate kernel (GEMM alone 9.55 ms) and 15.0 ms for a 32x32x16 kernel with
 // one barrier per 32-wide step; 1024 -> 2 x 4096 on 294,912 rows 3.86 against 5.27 ms; one member
-// (49,152 rows) 398 against 602 us.
+// (49,152 rows) 389 against 602 us.
 #include "bsa_common.h"
 #include "mosaic_bsa.h"
 
@@ -38,7 +39,7 @@ constexpr int kHid = 128;            // hidden indices per tile
 constexpr int kK = 64;               // reduction step of an iteration
 constexpr int kHalf = 128 * kK;      // elements of an operand half in LDS: 128 rows of 128 bytes
 constexpr int kStage = 32 * 32;      // elements of a wave's output staging (a 32 x 32 piece)
-constexpr int kNoiseRows = 56;       // noise rows staged in LDS (what the 160 KB leave)
+constexpr int kNoiseRows = 56;       // noise rows staged in LDS (the 160 KB would leave 64)
 constexpr int kStores = 8;           // global stores of a wave per tile
 constexpr int kWorkgroups = 256;     // one per CU
 
@@ -71,10 +72,18 @@ template <int N>
 __device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory"); }
 __device__ __forceinline__ void barrier() { asm volatile("s_barrier" ::: "memory"); }
 
-// bf16(silu(a)) * b in fp32
+// bf16(silu(a)) * b in fp32, for a bf16 value a: a / (1 + exp(-a)) as (a / 4) / (1/4 + exp(-a) / 4).
+// For every one of the 65,536 arguments the bf16 value is that of expf and a correctly rounded
+// division, which take about 20 vector instructions against these 4: the rounding of a log2 e grows to
+// 55 fp32 spacings of the result at a = -88 (3 for |a| < 4), a bf16 spacing is 65,536 of them, and
+// no argument's result is that near to where the rounding changes.  The quarters keep the
+// reciprocal out of the subnormal range, which the hardware flushes (a from -88.5 to -87.5).  The
+// addend is one spacing above 1/4: with 1/4 itself one argument, 5.9375, rounds the other way.
+// 768 -> 2 x 3072 on 1,179,648 rows: 9.40 ms; a rcp(1 + exp2(a * -log2 e)), which is wrong for
+// these four arguments, 9.28 ms.
 __device__ __forceinline__ float gate(float a, float b) {
-    const float e = __builtin_amdgcn_exp2f(a * -1.44269504088896f);
-    return round_bf16(a * __builtin_amdgcn_rcpf(1.0f + e)) * b;
+    const float e = __builtin_amdgcn_exp2f(fmaf(a, -1.44269504088896f, -2.0f));
+    return round_bf16(a * 0.25f * __builtin_amdgcn_rcpf(e + 0.25000003f)) * b;
 }
 
 // Where a row's noise comes from: none, its slice of the tile's columns staged in LDS (up to

@@ -179,3 +179,27 @@ def test_cswiglu_routes(change, monkeypatch):
     assert n == (1 if change == "none" else 0) and len(calls) == n
     assert len(seen) == (2 if "hook" in change else 0)
     check(got, want, change)
+
+
+def test_swiglu_linear_gate_every_argument():
+    """silu of every bf16 value (negative zero aside: a sum of products has none), subnormal, infinite
+    and NaN ones among them, each as one product 1 * value: the bits of the gate kernel (expf and a
+    division), and where the float64 silu is a normal value, its bf16 rounding."""
+    hidden, dim = 65536, 128
+    values = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    values[values == 0] = 0.0
+    x = torch.zeros(256, 1, dim, dtype=torch.bfloat16)
+    x[..., 0] = 1.0
+    w13 = torch.zeros(2 * hidden, dim, dtype=torch.bfloat16)
+    w13[:hidden, 0] = values
+    w13[hidden:, 0] = 1.0
+    got = fused.swiglu_linear_w13(x.to(DEV), w13.to(DEV))[[0, 255], 0].cpu()
+    h = torch.cat([values, torch.ones_like(values)]).to(DEV).expand(2, 1, -1).contiguous()
+    want = fused.swiglu(h)[:, 0].cpu()
+    nan = want.isnan()
+    assert torch.equal(got.isnan(), nan)
+    assert torch.equal(got.view(torch.int16)[~nan], want.view(torch.int16)[~nan])
+    a = values.double()
+    exact = a / (1 + torch.exp(-a))
+    normal = exact.isfinite() & (exact.abs() >= 2.0 ** -126) & (a > -88.7)   # below, expf overflows: -0
+    assert normal.sum() > 64000 // 2 and torch.equal(got[:, normal], exact[normal].to(torch.bfloat16).expand(2, -1))
