@@ -24,6 +24,8 @@ from dataclasses import dataclass
 
 import torch
 import torch.nn as nn
+import torch.nn.functional as F
+from torch.utils._device import DeviceContext
 
 from . import fused
 from .fused import RMSNorm
@@ -134,6 +136,23 @@ def era5_config(num_variables: int = 82, num_static: int = 3) -> ModelConfig:
         noise_dim=32, rmsnorm_elementwise_affine=False)
 
 
+_LINEAR_FORWARD, _F_LINEAR = nn.Linear.forward, F.linear
+
+
+def _plain_linear(lin: nn.Module) -> bool:
+    """Whether calling ``lin`` is torch's own product with ``lin.weight`` and nothing else sees or
+    replaces it: no other class, parameter type, bias or hook, no ``forward`` assigned to the module
+    (as libraries that offload, quantise or adapt a Linear do), to its class or to ``F.linear``, no
+    compiled call, and no dispatch or function mode that watches the product (a default device aside)."""
+    return (type(lin) is nn.Linear and type(lin.weight) is nn.Parameter and lin.bias is None
+            and "forward" not in lin.__dict__ and "_call_impl" not in lin.__dict__ and lin._compiled_call_impl is None
+            and nn.Linear.forward is _LINEAR_FORWARD and F.linear is _F_LINEAR
+            and not (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks or lin._backward_pre_hooks)
+            and not nn.modules.module._has_any_global_hook()
+            and torch._C._len_torch_dispatch_stack() == 0
+            and all(type(m) is DeviceContext for m in torch.overrides._get_current_function_mode_stack()))
+
+
 class cSwiGLU(nn.Module):
     """SwiGLU feed-forward with an additive noise bias on the gate (primitives.py:92-105):
     ``w2(silu(x1 + noise_bias(z)) * x3)`` with ``x1, x3 = w13(x).chunk(2)``."""
@@ -153,13 +172,10 @@ class cSwiGLU(nn.Module):
     fused_linear_gate = True
 
     def _one_kernel(self, x: torch.Tensor, noise: torch.Tensor | None) -> torch.Tensor | None:
-        """w13 and the gate as one kernel, or None where they run as two: w13 replaced, hooked or
-        biased, arithmetic other than bf16, or a shape the kernel does not take."""
+        """w13 and the gate as one kernel, or None where they run as two: w13 not a plain Linear
+        (``_plain_linear``), arithmetic other than bf16, or a shape the kernel does not take."""
         lin = self.w13
-        if (type(lin) is not nn.Linear or type(lin.weight) is not nn.Parameter or lin.bias is not None
-                or type(x) is not torch.Tensor or not x.is_cuda or x.dtype != torch.bfloat16
-                or lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks or lin._backward_pre_hooks
-                or torch.nn.modules.module._has_any_global_hook()):
+        if type(x) is not torch.Tensor or not x.is_cuda or x.dtype != torch.bfloat16 or not _plain_linear(lin):
             return None
         forward_only("cSwiGLU", x, lin.weight, noise)
         if torch.is_autocast_enabled("cuda"):

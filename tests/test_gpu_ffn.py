@@ -1,9 +1,13 @@
 """cSwiGLU's w13 projection and gate as one kernel (fused.swiglu_linear, ffn.hip) against the
 reference's two steps (primitives.py:92-105): h = x w13^T as a bf16 Linear (fp32
 accumulation, rounded to bf16), then the gate with the eager bf16 rounding points."""
+import contextlib
+
 import pytest
 import torch
 import torch.nn.functional as F
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from mosaic_amd import fused
 from mosaic_amd.model import cSwiGLU
@@ -139,7 +143,31 @@ def test_swiglu_linear_w13_non_finite_rows_stay_in_their_rows():
     assert torch.equal(got[5].isnan(), want[0].isnan()) and torch.equal(got[5].isinf(), want[0].isinf())
 
 
-@pytest.mark.parametrize("change", ["none", "hook", "global_hook", "bias", "replaced", "fp32_noise", "odd_rows", "view"])
+class _SeenFunctions(TorchFunctionMode):
+    def __init__(self, seen):
+        super().__init__()
+        self.seen = seen
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        if func is F.linear and args[1].shape[0] == 2048:
+            self.seen.append(1)
+        return func(*args, **(kwargs or {}))
+
+
+class _SeenOperators(TorchDispatchMode):
+    def __init__(self, seen):
+        super().__init__()
+        self.seen = seen
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        if func in (torch.ops.aten.mm.default, torch.ops.aten.addmm.default) and args[-1].shape[-1] == 2048:
+            self.seen.append(1)
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("change", ["none", "default_device", "hook", "global_hook", "bias", "replaced", "fp32_noise",
+                                    "odd_rows", "view", "forward", "class_forward", "linear", "compiled",
+                                    "function_mode", "dispatch_mode"])
 def test_cswiglu_routes(change, monkeypatch):
     """The module takes the one kernel only where nothing observes or replaces w13 and the shape
     fits, and its result is the two-step one on every route."""
@@ -150,7 +178,24 @@ def test_cswiglu_routes(change, monkeypatch):
     calls, seen = [], []
     real = fused.swiglu_linear_w13
     monkeypatch.setattr(fused, "swiglu_linear_w13", lambda *a: calls.append(1) or real(*a))
-    handle = None
+    handle, mode = None, contextlib.nullcontext()
+    if change == "forward":
+        own = m.w13.forward
+        m.w13.forward = lambda t: seen.append(1) or own(t)
+    elif change == "class_forward":
+        base = torch.nn.Linear.forward
+        monkeypatch.setattr(torch.nn.Linear, "forward", lambda lin, t: (lin is m.w13 and seen.append(1)) or base(lin, t))
+    elif change == "linear":
+        base = F.linear
+        monkeypatch.setattr(F, "linear", lambda t, w, b=None: (w is m.w13.weight and seen.append(1)) or base(t, w, b))
+    elif change == "compiled":
+        m.w13._compiled_call_impl = lambda t: seen.append(1) or F.linear(t, m.w13.weight)
+    elif change == "function_mode":
+        mode = _SeenFunctions(seen)
+    elif change == "dispatch_mode":
+        mode = _SeenOperators(seen)
+    elif change == "default_device":
+        mode = torch.device(DEV)
     if change == "hook":
         m.w13.register_forward_hook(lambda *a: seen.append(1))
     elif change == "global_hook":
@@ -169,15 +214,16 @@ def test_cswiglu_routes(change, monkeypatch):
     elif change == "view":
         x = torch.randn(1030, 2, 512, device=DEV).to(torch.bfloat16)[..., 128:384]
     try:
-        with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16), mode:
             got = m(x, z)
             n, m.fused_linear_gate = len(calls), False
             want = m(x, z)
     finally:
         if handle is not None:
             handle.remove()
-    assert n == (1 if change == "none" else 0) and len(calls) == n
-    assert len(seen) == (2 if "hook" in change else 0)
+    assert n == (1 if change in ("none", "default_device") else 0) and len(calls) == n
+    watched = ("hook", "global_hook", "forward", "class_forward", "linear", "compiled", "function_mode", "dispatch_mode")
+    assert len(seen) == (2 if change in watched else 0)
     check(got, want, change)
 
 
