@@ -185,7 +185,9 @@ class cSwiGLU(nn.Module):
             return None
         if x.dim() < 2 or not fused.swiglu_linear_pays(x.numel() // max(1, x.shape[-1]), lin.out_features // 2):
             return None
-        w = lin.weight.to(torch.bfloat16)
+        # One operand and nothing to contract: the weight itself, or under autocast its cast as w13
+        # would take it, from autocast's cache where that holds it (a .to() would cast at every call).
+        w = torch.einsum("ij->ij", lin.weight)
         return fused.swiglu_linear_w13(x, w, noise) if fused.swiglu_linear_w13_ok(x, w, noise) else None
 
     def forward(self, x: torch.Tensor, z: torch.Tensor | None = None) -> torch.Tensor:

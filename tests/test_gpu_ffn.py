@@ -165,6 +165,15 @@ class _SeenOperators(TorchDispatchMode):
         return func(*args, **(kwargs or {}))
 
 
+class _Casts(TorchDispatchMode):
+    """Counts the casts of a 2048-row weight to bf16."""
+    n = 0
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.n += func is torch.ops.aten._to_copy.default and args[0].shape[0] == 2048 and args[0].dtype == torch.float32
+        return func(*args, **(kwargs or {}))
+
+
 @pytest.mark.parametrize("change", ["none", "default_device", "hook", "global_hook", "bias", "replaced", "fp32_noise",
                                     "odd_rows", "view", "forward", "class_forward", "linear", "compiled",
                                     "function_mode", "dispatch_mode"])
@@ -225,6 +234,25 @@ def test_cswiglu_routes(change, monkeypatch):
     watched = ("hook", "global_hook", "forward", "class_forward", "linear", "compiled", "function_mode", "dispatch_mode")
     assert len(seen) == (2 if change in watched else 0)
     check(got, want, change)
+
+
+@pytest.mark.parametrize("cache,frozen", [(True, False), (False, False), (True, True)])
+def test_cswiglu_weight_cast_is_autocasts(cache, frozen, monkeypatch):
+    """Inside one autocast region w13 is cast as often as its Linear would: once where autocast
+    caches the cast, at every call with its cache off or a weight that needs no gradient."""
+    m = cSwiGLU(256, 1024, 0).to(DEV).requires_grad_(not frozen)
+    x = torch.randn(2048, 1, 256, device=DEV).to(torch.bfloat16)
+    weights = []
+    real = fused.swiglu_linear_w13
+    monkeypatch.setattr(fused, "swiglu_linear_w13", lambda x, w, n: weights.append(w) or real(x, w, n))
+    linear_casts = _Casts()
+    with torch.no_grad():
+        with torch.autocast("cuda", dtype=torch.bfloat16, cache_enabled=cache):
+            m(x), m(x)
+        with torch.autocast("cuda", dtype=torch.bfloat16, cache_enabled=cache), linear_casts:
+            m.w13(x), m.w13(x)
+    assert len(weights) == 2 and all(w.dtype == torch.bfloat16 for w in weights)
+    assert len({w.data_ptr() for w in weights}) == linear_casts.n == (1 if cache and not frozen else 2)
 
 
 def test_swiglu_linear_gate_every_argument():
