@@ -305,7 +305,7 @@ void swiglu_linear_kernel(SwigluLinearParams p) {
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
                     const int row = 16 * i + (lane >> 2), c = lane & 3;
-                    *reinterpret_cast<uint4*>(ob + (uint32_t)(2 * ((piece + row) * p.hidden + 8 * c))) =
+                    *reinterpret_cast<uint4*>(ob + 2 * ((int64_t)(piece + row) * p.hidden + 8 * c)) =
                         *reinterpret_cast<const uint4*>(stg + row * 32 + 8 * (c ^ ((row >> 2) & 3)));
                 }
                 __builtin_amdgcn_wave_barrier();
@@ -332,9 +332,8 @@ int swiglu_linear(const void* x, int64_t rows, int32_t dim, int64_t x_row_stride
     if (x_row_stride < dim || x_row_stride % 8) return MOSAIC_ERR_ALIGNMENT;
     if (!aligned16(x) || !aligned16(weight) || !aligned16(out) || (noise && !aligned16(noise)))
         return MOSAIC_ERR_ALIGNMENT;
-    // byte offsets within a wave's 16 rows of x or w13, within a tile of out and within the staged
-    // noise are 32-bit
-    if (x_row_stride >= ((int64_t)1 << 26) || dim >= (1 << 26) || hidden >= (1 << 22)) return MOSAIC_ERR_UNSUPPORTED;
+    // byte offsets within a wave's 16 rows of x or w13 are 32-bit
+    if (x_row_stride >= ((int64_t)1 << 26) || dim >= (1 << 26)) return MOSAIC_ERR_UNSUPPORTED;
     const int64_t row_tiles = (rows + kM - 1) / kM, n_tiles = hidden / kHid;
     if (row_tiles > 0x7fffffff / n_tiles / 8) return MOSAIC_ERR_SHAPE;
     SwigluLinearParams p{};
@@ -360,8 +359,9 @@ int swiglu_linear(const void* x, int64_t rows, int32_t dim, int64_t x_row_stride
     // zero operands, 294,912 rows, dim 768: 1718 against 1832 us at 4; dim 3072: 5680 against 5420.
     p.group_rows = dim <= 1024 ? 8 : 4;
     const void* fn = !noise ? (const void*)&swiglu_linear_kernel<kNoNoise>
-                   : noise_rows <= kNoiseRows ? (const void*)&swiglu_linear_kernel<kNoiseLds>
-                                              : (const void*)&swiglu_linear_kernel<kNoiseGlobal>;
+                   : noise_rows <= kNoiseRows && hidden < (1 << 25)  // byte offsets of the staged rows are 32-bit
+                       ? (const void*)&swiglu_linear_kernel<kNoiseLds>
+                       : (const void*)&swiglu_linear_kernel<kNoiseGlobal>;
     const int grid = p.tiles >= kWorkgroups ? kWorkgroups : (p.tiles + 7) / 8 * 8;
     void* args[] = {&p};
     const hipError_t e = hipLaunchKernel(fn, dim3(grid), dim3(512), args, 0, static_cast<hipStream_t>(stream));

@@ -70,6 +70,19 @@ def test_swiglu_linear_strided_rows():
     check(got, reference(x, w13, None), "strided x")
 
 
+def test_swiglu_linear_wide_hidden():
+    """A tile of out that spans more than 4 GB: byte offsets past 32 bits, every row and noise row."""
+    hidden, dim = (1 << 23) + (1 << 16), 128
+    g = torch.Generator(DEV).manual_seed(8)
+    x = torch.randn(128, 2, dim, generator=g, device=DEV).to(torch.bfloat16)
+    w13 = torch.empty(2 * hidden, dim, dtype=torch.bfloat16, device=DEV).normal_(0, dim ** -0.5, generator=g)
+    nz = torch.empty(2, hidden, dtype=torch.bfloat16, device=DEV).normal_(generator=g)
+    got = fused.swiglu_linear(x, fused.permute_w13(w13), nz)
+    cols = torch.cat([torch.arange(c, c + 256) for c in (0, hidden // 2, hidden - 256)]).to(DEV)
+    ref = reference(x, torch.cat([w13[cols], w13[hidden + cols]]), nz[:, cols])
+    check(got[..., cols], ref, "wide hidden")
+
+
 def test_cswiglu_module_fused_equals_unfused():
     """cSwiGLU.forward through the fused kernel and through w13 + gate kernel + w2."""
     torch.manual_seed(0)
