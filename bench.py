@@ -549,8 +549,11 @@ def main():
     ap.add_argument("--unet-warmup", type=int, default=1)
     ap.add_argument("--unet-fused-input-side", action="store_true",
                     help="U-Net attention blocks take the fused projection kernel (mosaic_attn_proj)")
-    ap.add_argument("--unet-two-step-ffn", action="store_true",
-                    help="U-Net feed-forward blocks run w13 as a library GEMM and the SwiGLU gate as its own kernel")
+    ffn = ap.add_mutually_exclusive_group()
+    ffn.add_argument("--unet-two-step-ffn", action="store_true",
+                     help="U-Net feed-forward blocks run w13 as a library GEMM and the SwiGLU gate as its own kernel")
+    ffn.add_argument("--unet-fused-ffn", action="store_true",
+                     help="U-Net feed-forward blocks run w13 and the SwiGLU gate as one kernel (the default)")
     ap.add_argument("--calibration-copy-mb", type=int, default=0,
                     help="after timing, run one device-to-device copy of this many MiB (a known-size "
                          "kernel for scaling FETCH_SIZE / WRITE_SIZE counters)")

@@ -41,3 +41,12 @@ def test_more_than_one_gpu_is_refused():
     assert r.returncode == 2
     assert "one GPU" in r.stderr
     assert r.stdout == ""
+
+
+def test_ffn_flags():
+    """Both forms of the feed-forward can be named; no flag means one kernel."""
+    for flags, ok in (([], True), (["--unet-fused-ffn"], True), (["--unet-two-step-ffn"], True),
+                      (["--unet-fused-ffn", "--unet-two-step-ffn"], False)):
+        r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2", *flags], capture_output=True,
+                           text=True)
+        assert r.returncode == 2 and ("one GPU only" in r.stderr) == ok, r.stderr
