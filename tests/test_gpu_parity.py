@@ -473,13 +473,14 @@ def test_mosaic_attention_module_runs():
 
 
 @pytest.mark.parametrize("B,N,H,bs", [
-    (1, 192, 1, 64), (1, 3072, 5, 64), (2, 1536, 3, 128), (1, 2048, 2, 1024), (1, 600, 3, 24), (1, 1400, 7, 200),
-    (1, 24576, 12, 64), (1, 49152, 18, 64), (12, 49152, 16, 64)],
-    ids=["one_head", "small", "bs128", "bs1024", "bs24", "bs200", "four_threads", "one_thread", "largest"])
+    (1, 192, 1, 64), (1, 8192, 18, 64), (1, 12288, 18, 64), (1, 49152, 18, 64), (2, 49152, 18, 64), (12, 49152, 16, 64),
+    (2, 1536, 3, 128), (1, 2048, 2, 1024), (1, 72, 3, 8), (1, 600, 3, 24), (1, 400, 3, 40), (1, 216, 3, 72),
+    (1, 1400, 7, 200), (64, 7280, 18, 104), (1, 64, 270000, 64)],
+    ids=["8_threads", "4_threads", "2_threads", "2_threads_wg64", "4_threads_mid", "8_threads_largest", "bs128", "bs1024",
+         "bs8", "bs24", "bs40", "bs72", "bs200", "bs104_largest", "most_workgroups"])
 def test_pool_mean_thread_splits(B, N, H, bs):
-    """Every split of a block's token walk (1, 2, 4 and 8 threads per column chunk; runs of
-    unequal length at 24 and 200 tokens): within half a bf16 spacing (2^-8 relative) of the
-    float64 mean, plus the fp32 sum's bound bs 2^-24 mean|x|."""
+    """Every split of a block's token walk (2, 4 and 8 threads per column chunk, each with its workgroups)
+    and blocks whose runs are unequal or empty: within half a bf16 spacing (2^-8 relative) of the float64 mean, plus the fp32 sum's bound bs 2^-24 mean|x|."""
     print(f"pool split B={B} N={N} H={H} bs={bs}", flush=True)
     x = torch.randn(B, N, H, 64, generator=torch.Generator(DEV).manual_seed(N + bs), device=DEV).to(torch.bfloat16)
     got = M.pool_mean(x, bs)
@@ -487,3 +488,39 @@ def test_pool_mean_thread_splits(B, N, H, bs):
     ref = blocks.mean(2, dtype=torch.float64)
     bound = 2 ** -8 * ref.abs() + bs * 2 ** -24 * blocks.abs().mean(2, dtype=torch.float64)
     assert got.shape == ref.shape and ((got.double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("bs", [16, 24, 40, 64, 72, 128])
+def test_pool_mean_of_a_member_alone_and_in_an_ensemble(bs):
+    """A member's pooled means do not depend on how many members (here 1 to 64: every thread split)
+    or heads the call has: the same bits, where the order of the sum shows (values from 2^-16 to 2^16)."""
+    print(f"pool alone / ensemble bs={bs}", flush=True)
+    g = torch.Generator(DEV).manual_seed(bs)
+    x = torch.randn(64, 48 * bs, 18, 64, generator=g, device=DEV)
+    x = x.mul_(torch.exp2(torch.randint(-16, 17, x.shape, generator=g, device=DEV).float())).to(torch.bfloat16)
+    every = M.pool_mean(x, bs)
+    for n in (1, 2, 4, 8, 24):
+        assert torch.equal(M.pool_mean(x[:n], bs), every[:n]), n
+    assert torch.equal(M.pool_mean(x[:1, :, :1], bs), every[:1, :, :1])
+
+
+@pytest.mark.parametrize("B,nside,Hq,Hk,bl,bs,K", [
+    (1, 32, 16, 4, 1024, 128, 12), (1, 64, 12, 3, 64, 64, 8), (1, 64, 12, 3, 1024, 128, 24), (6, 64, 12, 3, 1024, 128, 8),
+    (1, 32, 8, 2, 512, 512, 4)], ids=["8_threads", "2_threads", "4_threads", "8_threads_wg512", "global_tables"])
+def test_fused_rope_every_pooling_split(B, nside, Hq, Hk, bl, bs, K):
+    """Each thread split of the pooling pass with RoPE, its table rows staged or read from global memory: the
+    rotated rows equal the rotation, and selections and output those of the plain op on them, whose
+    pooling splits otherwise."""
+    print(f"rope split B={B} nside={nside} bs={bs}", flush=True)
+    g = torch.Generator(DEV).manual_seed(nside + bs)
+    q, k, v = (torch.randn(B, 12 * nside ** 2, h, 64, generator=g, device=DEV) for h in (Hq, Hk, Hk))
+    q, k = (t.mul_(torch.exp2(torch.randint(-12, 2, t.shape, generator=g, device=DEV).float())) for t in (q, k))
+    q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
+    w = torch.softmax(torch.randn(3, B, 12 * nside ** 2, Hq, 1, generator=g, device=DEV), 0).to(torch.bfloat16)
+    cos, sin = (t.to(DEV) for t in rope_tables(get_healpix_grid(nside), 64))
+    out, q_rot, k_rot, idx = M.mosaic_attn_func_rope(q, k, v, w, cos, sin, bl, bs, K, False, return_rotated=True,
+                                                     return_block_indices=True)
+    assert torch.equal(q_rot[:1].cpu(), apply_rope(q[:1].cpu(), cos.cpu(), sin.cpu()))
+    assert torch.equal(k_rot[-1:].cpu(), apply_rope(k[-1:].cpu(), cos.cpu(), sin.cpu()))
+    ref_out, ref_idx = M.mosaic_attn_func(q_rot, k_rot, v, w, bl, bs, K, False, return_block_indices=True)
+    assert torch.equal(idx, ref_idx) and torch.equal(out, ref_out)
