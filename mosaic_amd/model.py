@@ -144,13 +144,15 @@ def _plain_linear(lin: nn.Module) -> bool:
     replaces it: no other class, parameter type, bias or hook, no ``forward`` assigned to the module
     (as libraries that offload, quantise or adapt a Linear do), to its class or to ``F.linear``, no
     compiled call, and no dispatch or function mode that watches the product (a default device aside)."""
-    return (type(lin) is nn.Linear and type(lin.weight) is nn.Parameter and lin.bias is None
-            and "forward" not in lin.__dict__ and "_call_impl" not in lin.__dict__ and lin._compiled_call_impl is None
+    own = lin.__dict__
+    return (type(lin) is nn.Linear and "forward" not in own and "_call_impl" not in own and lin._compiled_call_impl is None
+            and type(own["_parameters"].get("weight")) is nn.Parameter and own["_parameters"].get("bias") is None
             and nn.Linear.forward is _LINEAR_FORWARD and F.linear is _F_LINEAR
-            and not (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks or lin._backward_pre_hooks)
+            and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"])
             and not nn.modules.module._has_any_global_hook()
             and torch._C._len_torch_dispatch_stack() == 0
-            and all(type(m) is DeviceContext for m in torch.overrides._get_current_function_mode_stack()))
+            and (torch._C._len_torch_function_stack() == 0
+                 or all(type(m) is DeviceContext for m in torch.overrides._get_current_function_mode_stack())))
 
 
 class cSwiGLU(nn.Module):
