@@ -907,18 +907,39 @@ hipError_t launch_knn_attn(const InterpParams& p, hipStream_t s) {
 // launch_knn_attn otherwise).
 bool knn_tiled_supported(const InterpParams& p) { return !p.round_products && knn_off32(p); }
 
+// Heads per workgroup of the tiled kernel, for a chip with room for slots workgroups at a time.  A
+// workgroup's time is its passes (heads times members) and a prologue, the tables' chained loads,
+// worth one and a half; the choice is the least product of that with the rounds of workgroups
+// (whole ones up to two, above that with a quarter for the uneven end) among groups of at most 48
+// passes, above which the prologue no longer counts.  Over 120 shapes (205 to 3878 tiles, 64 to
+// 128 rows, 8 to 32 neighbours, 4 to 20 heads, 1 to 24 members) it is within 7 % of the fastest
+// group, 0.6 % on average.  us at one head, at the fastest group, at the choice: 3878 tiles, 12 heads,
+// one member 332, 194 (12 heads), 194; 24 members 2571, 2469 (3), 2488 (2); 837 tiles of 128 rows,
+// 4 heads, one member 43, 32 (4), 32; 205 tiles of 128 rows, 12 heads, one member 31.7, 24.5 (6), 24.5.
+static int heads_per_workgroup(int64_t tiles, int H, int B, int slots) {
+    int best = 1;
+    double least = 0.;
+    for (int h = 1; h <= H && (h == 1 || (int64_t)h * B <= 48); ++h) {
+        const int groups = (H + h - 1) / h, hg = (H + groups - 1) / groups;  // groups as equal as they get
+        const double rounds = (double)(tiles * groups) / slots, whole = ceil(rounds);
+        const double cost = (whole <= 2. ? whole : rounds + 0.25) * (1.5 + (double)hg * B);
+        if (h == 1 || cost < least) {
+            least = cost;
+            best = hg;
+        }
+    }
+    return best;
+}
+
 hipError_t launch_knn_attn_tiled(const InterpParams& p, const KnnTiles& t, hipStream_t s) {
     if (!knn_tiled_supported(p) || t.rows <= 0 || t.rows % 8 || t.rows > kKnnTileRows) return hipErrorInvalidValue;
-    // heads per workgroup: 48 passes (heads times members) make a workgroup's prologue (the
-    // tables, 4 us of chained loads) small, but 2048 workgroups are left to fill the chip's 768
-    // slots evenly (the model's grids, 12 heads: one member 218 us at 1 head, 120 at 12; 24
-    // members 2604 at 1, 2469 at 2, 2678 at 12; 563 tiles, 4 heads, 24 members: 179 at 1 head,
-    // 191 at 2); a grid smaller than that takes one round of the slots (68 tiles, 12 heads, one
-    // member: 28 us at 1 head, 21 at 2)
-    const int64_t work = (int64_t)t.n * p.H;
-    const int64_t fill = work < 2048 ? (work + 767) / 768 : work / 2048;
-    int hg = (int)max((int64_t)1, min(min((int64_t)(48 + p.B - 1) / p.B, fill), (int64_t)p.H));
-    hg = (p.H + (p.H + hg - 1) / hg - 1) / ((p.H + hg - 1) / hg);  // groups as equal as they get
+    // per row: k and v, two buffers each; then the waves' tables (12 bytes per target and
+    // neighbour)
+    const size_t lds = 512u * (size_t)t.rows + (size_t)kKnnTileTargets * 8u * ((p.K + 7) / 8) * 12u;
+    // three workgroups per CU; two from 25 neighbours on (compiled for two waves per SIMD) and where
+    // the LDS holds no third
+    const int per_cu = (int)min((size_t)(p.K > 24 ? 2 : 3), (size_t)163840 / lds);
+    int hg = heads_per_workgroup(t.n, p.H, p.B, 256 * per_cu);
     const int64_t wgs = (int64_t)t.n * ((p.H + hg - 1) / hg);
     if (wgs <= 0) return hipSuccess;
     if (wgs > 0x7fffffff) return hipErrorInvalidValue;
@@ -931,9 +952,6 @@ hipError_t launch_knn_attn_tiled(const InterpParams& p, const KnnTiles& t, hipSt
         case 4: fn = p.scale_pow2 ? (const void*)&knn_tile_kernel<4, true> : (const void*)&knn_tile_kernel<4, false>; break;
         default: return hipErrorInvalidValue;
     }
-    // per row: k and v, two buffers each; then the waves' tables (12 bytes per target and
-    // neighbour)
-    const size_t lds = 512u * (size_t)t.rows + (size_t)kKnnTileTargets * 8u * ((p.K + 7) / 8) * 12u;
     return hipLaunchKernel(fn, dim3((unsigned)wgs), dim3(kTileWaves * 64), args, lds, s);
 }
 
