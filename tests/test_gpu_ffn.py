@@ -95,7 +95,7 @@ def test_cswiglu_module_fused_equals_unfused():
         m.fused_linear_gate = False
         b = m(x, z)
     check(a, b, "module fused vs unfused")
-    # the permuted weight is rebuilt when the weight changes
+    # a changed weight is seen by the next region
     with torch.no_grad():
         m.w13.weight.mul_(0.5)
         m.fused_linear_gate = True
@@ -134,9 +134,13 @@ def test_swiglu_linear_w13_shapes(S, B, dim, hidden, noise):
     x = torch.randn(S, B, dim, generator=g).to(torch.bfloat16)
     w13 = (torch.randn(2 * hidden, dim, generator=g) * dim ** -0.5).to(torch.bfloat16)
     nz = torch.randn(B, hidden, generator=g).to(torch.bfloat16) if noise else None
-    torch.full((S, B, hidden), float("nan"), dtype=torch.bfloat16, device=DEV)   # freed: the next output's memory
-    with torch.no_grad():
-        got = fused.swiglu_linear_w13(x.to(DEV), w13.to(DEV), nz.to(DEV) if noise else None)
+    xd, wd, nd = x.to(DEV), w13.to(DEV), nz.to(DEV) if noise else None
+    torch.cuda.empty_cache()
+    poison = torch.full((S, B, hidden), float("nan"), dtype=torch.bfloat16, device=DEV)
+    memory = poison.data_ptr()
+    del poison                                   # the next output's memory
+    got = fused.swiglu_linear_w13(xd, wd, nd)
+    assert got.data_ptr() == memory
     ref = reference(x, w13, nz)
     check(got, ref, "vs fp32-accumulate reference")
     # only sums in another order and the silu's last fp32 bits differ: bf16 roundings rarely flip
