@@ -42,6 +42,11 @@ constexpr int kStage = 32 * 32;      // elements of a wave's output staging (a 3
 constexpr int kNoiseRows = 56;       // noise rows staged in LDS (the 160 KB would leave 64)
 constexpr int kStores = 8;           // global stores of a wave per tile
 constexpr int kWorkgroups = 256;     // one per CU
+// Row tiles per group: the group's x rows stay in an XCD's L2 (4 MB) while the weights pass by, and a
+// longer group reads the weights less often.  Random operands, 294,912 rows, at 2, 4, 8 and 16 row
+// tiles: 1024 -> 2 x 4096 3878, 3801, 3804, 4052 us; 3072 -> 2 x 3072 7645, 7487, 7499, 7602; 1,179,648 rows,
+// 768 -> 2 x 3072 9419, 9244, 9249, 9331; 73,728 rows, 1280 -> 2 x 5120 1455, 1437, 1431, 1443.
+constexpr int kGroupRows = 8;
 
 struct SwigluLinearParams {
     const bf16_t* x;        // [rows, D], row stride x_sr (elements)
@@ -51,7 +56,7 @@ struct SwigluLinearParams {
     int64_t x_sr, rows;
     int64_t w_x3;           // rows from an x1 row to its x3 row
     int w_tile, w_wave1, w_wave2;   // weight row of wave w in a tile: (w / 2) * w_wave2 + (w % 2) * w_wave1
-    int D, hidden, noise_rows, n_tiles, row_tiles, tiles, group_rows;
+    int D, hidden, noise_rows, n_tiles, row_tiles, tiles;
     uint32_t noise_magic;   // ceil(2^32 / noise_rows): x / noise_rows as a high product
 };
 
@@ -106,14 +111,14 @@ void swiglu_linear_kernel(SwigluLinearParams p) {
     const int tbeg = xcd * per + min(xcd, rem), tend = tbeg + per + (xcd < rem ? 1 : 0);
     int tile = tbeg + slot;
     if (tile >= tend) return;  // the whole workgroup, before any barrier
-    // tiles in groups of group_rows row tiles, the row tile varying fastest inside a group
+    // tiles in groups of kGroupRows row tiles, the row tile varying fastest inside a group
     int rt, nt;
     auto tile_of = [&](int t, int& row_tile, int& col_tile) __attribute__((always_inline)) {
-        const int per_group = p.group_rows * p.n_tiles;
+        const int per_group = kGroupRows * p.n_tiles;
         const int grp = t / per_group, within = t - grp * per_group;
-        const int rows_here = min(p.group_rows, p.row_tiles - grp * p.group_rows);
+        const int rows_here = min(kGroupRows, p.row_tiles - grp * kGroupRows);
         col_tile = within / rows_here;
-        row_tile = grp * p.group_rows + (within - col_tile * rows_here);
+        row_tile = grp * kGroupRows + (within - col_tile * rows_here);
     };
     // the last row tile of a ragged row count starts early and repeats rows of the one before
     auto first_row = [&](int row_tile) __attribute__((always_inline)) -> int64_t {
@@ -354,10 +359,6 @@ int swiglu_linear(const void* x, int64_t rows, int32_t dim, int64_t x_row_stride
     p.n_tiles = (int)n_tiles;
     p.row_tiles = (int)row_tiles;
     p.tiles = (int)(row_tiles * n_tiles);
-    // Row tiles per group: the group's x rows stay in an XCD's L2 (4 MB) while the weights pass
-    // by, and a longer group reads the weights less often.  8 up to dim 1024 (4 MB of x), 4 above:
-    // zero operands, 294,912 rows, dim 768: 1718 against 1832 us at 4; dim 3072: 5680 against 5420.
-    p.group_rows = dim <= 1024 ? 8 : 4;
     const void* fn = !noise ? (const void*)&swiglu_linear_kernel<kNoNoise>
                    : noise_rows <= kNoiseRows && hidden < (1 << 25)  // byte offsets of the staged rows are 32-bit
                        ? (const void*)&swiglu_linear_kernel<kNoiseLds>
