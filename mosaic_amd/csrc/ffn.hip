@@ -13,9 +13,10 @@
 // lane then holds one row and four consecutive hidden indices per accumulator, so noise is one
 // 8-byte read and the output four packed values.
 //
-// What bounds it: the board's power limit in the main loop (on all-zero operands it runs at 93%
-// of the 2.5 PFLOP/s matrix peak, 2340 TFLOP/s, on random ones at 1630-1660), then the vector
-// work of the gate between two tiles.  The choices that follow:
+// What bounds it: the board's power limit in the main loop (its marginal rate, from two dims: 2340
+// TFLOP/s on all-zero operands, 93% of the 2.5 PFLOP/s matrix peak, 1630-1660 on random ones), then the
+// vector work of the gate between two tiles: 1200 TFLOP/s over the whole kernel at dim 768, 1300 at
+// 1024, 1490 at 3072.  The choices that follow:
 //  - v_mfma_f32_16x16x32_bf16 instead of 32x32x16: it reads and writes the fp32 accumulators
 //    half as often per product, and under the power limit the same loop runs 1505 -> 1659 TFLOP/s;
 //  - ping-pong: the four waves of one row half run half a phase behind the others, so on every

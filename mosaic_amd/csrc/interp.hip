@@ -576,8 +576,8 @@ __global__ __launch_bounds__(kInterpWaves * 64) __attribute__((amdgpu_waves_per_
 // stage k, 2 and 3 v.  The arithmetic per (target, member, head) is the fp32-product form of
 // the kernel above in the same order, so both give the same bits.
 //
-// The bound is vector-instruction issue and LDS reads together (65 % and 61 % busy at 24
-// members), so the work per (target, member, head) is cut where it was the same in many lanes.
+// The bound is vector-instruction issue and LDS reads together (57 % each at 24 members, and
+// bank conflicts 22 % of the LDS cycles), so the work per (target, member, head) is cut where it was the same in many lanes.
 // Each wave takes a quarter of the tile's targets (up to 4) together:
 //   scores   lane 8 jg + dc, as above, holds chunk dc of neighbours jg + 8 i of every target;
 //            the sums over the 8 chunk lanes leave target dc % 4's scores in lane (jg, dc), so
