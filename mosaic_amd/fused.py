@@ -160,7 +160,8 @@ def swiglu_linear(x: torch.Tensor, w13_perm: torch.Tensor, noise: torch.Tensor |
     """``swiglu(x @ w13^T, noise)`` in one kernel: the projection (bf16 operands, fp32
     accumulation, rounded to bf16 as a bf16 Linear) and the gate with its rounding points.
     x: bf16 ``[..., dim]`` (rows sequence-first ``[S, B]`` when noise is given); w13_perm:
-    ``permute_w13(w13)`` in bf16; noise: ``[B, hidden]`` or None.  Returns ``[..., hidden]``."""
+    ``permute_w13(w13)`` in bf16; noise: ``[B, hidden]`` or None.  Returns ``[..., hidden]``.
+    For callers that hold the weight in that order; the model runs ``swiglu_linear_w13``."""
     forward_only("fused.swiglu_linear", x, w13_perm, noise)
     two_h, dim = w13_perm.shape
     hidden = two_h // 2
